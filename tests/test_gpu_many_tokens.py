@@ -1,0 +1,90 @@
+"""GPU: the many-token forms of the shared expert and the routers, through the
+C ABI, at the sizes where a tile, a grid or a dispatch rule ends."""
+import numpy as np
+import pytest
+
+from oracle import binding as B
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nh():
+    import nmoe_hip
+    return nmoe_hip
+
+
+@pytest.fixture(scope="module")
+def ctx(nh):
+    c = nh.Context(0, max_tokens=1100)
+    yield c
+    c.close()
+
+
+def q4_tensor(rng, rows, cols, sigma, offset):
+    """A q4 tensor whose biases are not -8 scale, and a device copy whose
+    parts start `offset` elements into their buffers (w 4-byte, scales and
+    biases 2-byte aligned)."""
+    w = rng.integers(0, 2 ** 32, size=(rows, cols // 8), dtype=np.uint32)
+    s = B.f32_to_bf16((rng.standard_normal((rows, cols // 64)) * sigma).astype(np.float32)).reshape(rows, -1)
+    b = B.f32_to_bf16((rng.standard_normal((rows, cols // 64)) * 8 * sigma).astype(np.float32)).reshape(rows, -1)
+    return w, s, b
+
+
+def device_copy(ctx, t, offset):
+    out = []
+    for a in t:
+        buf = ctx.alloc(a.nbytes + 16)
+        buf.upload(a, offset * a.itemsize)
+        out.append(buf.ptr + offset * a.itemsize)
+    return tuple(out)
+
+
+def dequant64(t):
+    w, s, b = t
+    q = ((w[..., None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(s.shape[0], s.shape[1], 64)
+    f = lambda v: B.bf16_to_f32(v).reshape(v.shape).astype(np.float64)
+    return (q * f(s)[..., None] + f(b)[..., None]).reshape(s.shape[0], -1)
+
+
+def tokens(rng, ctx, nh, xdt, ntok):
+    x = rng.standard_normal((ntok, 2048)).astype(np.float32)
+    if xdt == "f32":
+        return x, ctx.to_device(x), nh.F32
+    xb = B.f32_to_bf16(x)
+    return B.bf16_to_f32(xb).reshape(ntok, 2048), ctx.to_device(xb), nh.BF16
+
+
+# per-token kernels up to 35 tokens (1, 2 or 4 tokens a block); then 16-, 32-
+# and 64-token tiles, each with a ragged last tile and, for the largest, the
+# die-wise tile order (16 tiles and more)
+@pytest.mark.parametrize("xdt,ntok", [("f32", 4), ("bf16", 5), ("f32", 13), ("bf16", 35), ("f32", 36), ("bf16", 241),
+                                      ("f32", 257), ("bf16", 512), ("f32", 513), ("bf16", 1025)])
+def test_shared_expert_many_tokens(ctx, nh, xdt, ntok):
+    """shared_out and the score against the products in 64 bits (relative L2
+    within 1e-6: fp32 sums of 2,048 and 512 terms, each rounding 2^-24, stay
+    below 5e-7), a few tokens against the oracle, and nothing written past
+    the last token."""
+    rng = np.random.default_rng(1000 + ntok)
+    t = {n: q4_tensor(rng, r, c, s, 1) for n, (r, c, s) in
+         {"gate": (512, 2048, 0.004), "up": (512, 2048, 0.004), "down": (2048, 512, 0.008),
+          "score": (1, 2048, 0.004)}.items()}
+    desc = nh.Context.shared_expert_desc(*(device_copy(ctx, t[n], 1) for n in ("gate", "up", "down", "score")))
+    x, dx, dt = tokens(rng, ctx, nh, xdt, ntok)
+    guard = np.full(2048, 7.5, np.float32)
+    so, gr = ctx.alloc((ntok + 1) * 8192), ctx.alloc((ntok + 1) * 4)
+    so.upload(guard, ntok * 8192)
+    gr.upload(guard[:1], ntok * 4)
+    ctx._check(ctx.shared_expert(desc, dx, dt, ntok, so, gr))
+    got, got_g = so.download(np.float32, (ntok + 1, 2048)), gr.download(np.float32, ntok + 1)
+    assert np.array_equal(got[ntok], guard) and got_g[ntok] == 7.5
+    x64 = x.astype(np.float64)
+    g, u = x64 @ dequant64(t["gate"]).T, x64 @ dequant64(t["up"]).T
+    want = (g / (1 + np.exp(-g)) * u) @ dequant64(t["down"]).T
+    want_g = (x64 @ dequant64(t["score"]).T)[:, 0]
+    rel = lambda a, b: np.linalg.norm(a - b) / np.linalg.norm(b)
+    print(f"[shared] {xdt} {ntok} tokens: rel {rel(got[:ntok], want):.2e}, score {rel(got_g[:ntok], want_g):.2e}")
+    assert rel(got[:ntok], want) < 1e-6 and rel(got_g[:ntok], want_g) < 1e-6
+    pick = np.unique([0, ntok // 2, ntok - 1])
+    want_so, want_gr = B.shared_expert({n: t[n] for n in t}, x[pick])
+    assert rel(got[pick], want_so) < 2e-6 and rel(got_g[pick], want_gr) < 2e-6
