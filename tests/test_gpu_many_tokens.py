@@ -88,3 +88,49 @@ def test_shared_expert_many_tokens(ctx, nh, xdt, ntok):
     pick = np.unique([0, ntok // 2, ntok - 1])
     want_so, want_gr = B.shared_expert({n: t[n] for n in t}, x[pick])
     assert rel(got[pick], want_so) < 2e-6 and rel(got_g[pick], want_gr) < 2e-6
+
+
+# one row a wavefront up to 95 (q4: 191) tokens, then tiles of 16 x 16, 32 x 32
+# (from 257) and 32 x 64 (from 1,025), with ragged last tiles of tokens and experts
+@pytest.mark.parametrize("kind,xdt,ntok,ne", [
+    ("bf16", "f32", 96, 256), ("bf16", "bf16", 241, 250), ("bf16", "f32", 257, 256), ("bf16", "bf16", 290, 33),
+    ("bf16", "bf16", 1025, 256), ("bf16", "f32", 1041, 241), ("q4", "f32", 192, 256), ("q4", "bf16", 193, 256),
+    ("q4", "f32", 300, 17), ("q4", "bf16", 1025, 250)])
+def test_router_many_tokens_bit_exact(ctx, nh, kind, xdt, ntok, ne):
+    """The matrix form's logits bit for bit the few-token kernel's (the same
+    tokens 64 at a time) and, for a few tokens, the oracle's; subnormal, huge,
+    infinite and NaN tokens among them; nothing written past the last logit."""
+    rng = np.random.default_rng(ntok * 7 + ne)
+    if kind == "bf16":
+        w = B.f32_to_bf16((rng.standard_normal((ne, 2048)) * 0.02).astype(np.float32)).reshape(ne, 2048)
+        r = nh.Context.router_bf16(ctx.to_device(w), ne)
+    else:
+        t = q4_tensor(rng, ne, 2048, 0.004, 1)
+        r = nh.Context.router_q4(*device_copy(ctx, t, 1), ne)
+    x = rng.standard_normal((ntok, 2048)).astype(np.float32)
+    x[1] *= np.float32(1e-38)
+    x[2] *= np.float32(3e36)
+    x[3, 17], x[4, 900], x[5] = np.inf, np.nan, 0.0
+    if xdt == "bf16":
+        xb = B.f32_to_bf16(x)
+        x, dx, dt, size = B.bf16_to_f32(xb).reshape(ntok, 2048), ctx.to_device(xb), nh.BF16, 2
+    else:
+        dx, dt, size = ctx.to_device(x), nh.F32, 4
+    lg, ref = ctx.alloc(ntok * ne * 4 + 64), ctx.alloc(ntok * ne * 4)
+    lg.upload(np.full(16, 7.5, np.float32), ntok * ne * 4)
+    ctx._check(ctx.router_logits(r, dx, dt, ntok, lg))
+    for t0 in range(0, ntok, 64):
+        ctx._check(ctx.router_logits(r, dx.ptr + t0 * 2048 * size, dt, min(64, ntok - t0), ref.ptr + t0 * ne * 4))
+    got, want = lg.download(np.float32, (ntok, ne)), ref.download(np.float32, (ntok, ne))
+    assert np.array_equal(lg.download(np.float32, 16, ntok * ne * 4), np.full(16, 7.5, np.float32))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fine = ~np.isnan(want)
+    np.testing.assert_array_equal(got.view(np.uint32)[fine], want.view(np.uint32)[fine])
+    for tok in (0, 16, ntok - 1):
+        if kind == "bf16":
+            o = B.router_logits_bf16(w, x[tok])
+        else:
+            o, xt = np.zeros(ne, np.float32), np.ascontiguousarray(x[tok], np.float32)
+            B.oracle().orc_router_logits_q4(t[0].ctypes.data, t[1].ctypes.data, t[2].ctypes.data, xt.ctypes.data, ne,
+                                            2048, o.ctypes.data)
+        np.testing.assert_array_equal(got[tok].view(np.uint32), o.view(np.uint32))
