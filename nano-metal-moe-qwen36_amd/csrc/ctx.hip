@@ -72,8 +72,7 @@ extern "C" int nmoe_hip_create(int device, int max_tokens, nmoe_hip_ctx **out) {
         return NMOE_HIP_ENODEV;
     }
     extern int nmoe_grouped_init(nmoe_hip_ctx *);
-    extern int nmoe_shared_init(nmoe_hip_ctx *);
-    if (nmoe_grouped_init(ctx) != NMOE_HIP_OK || nmoe_shared_init(ctx) != NMOE_HIP_OK) {
+    if (nmoe_grouped_init(ctx) != NMOE_HIP_OK) {
         nmoe_hip_destroy(ctx);
         return NMOE_HIP_ENOMEM;
     }
@@ -97,7 +96,6 @@ extern "C" void nmoe_hip_destroy(nmoe_hip_ctx *ctx) {
     hipFree(ctx->idx);
     hipFree(ctx->w);
     hipFree(ctx->s_act);
-    hipFree(ctx->s_mm);
     hipFree(ctx->sync);
     hipFree(ctx->xch);
     extern void nmoe_grouped_free(nmoe_hip_ctx *);

@@ -493,8 +493,7 @@ __global__ void __launch_bounds__(256, 2) nmoe_shared_mm_kernel(nmoe_sh_ws ws, i
  * 22 at 37. */
 #define NMOE_SHARED_MM_MIN 36
 
-/* Scratch of the matrix-core launches (none for a context of fewer tokens):
- * one allocation, every part a multiple of 1 KB. */
+/* Scratch of the matrix-core launches, every part a multiple of 1 KB. */
 static size_t nmoe_sh_layout(size_t max_tokens, uint8_t *base, nmoe_sh_ws *ws) {
     const size_t tb = (max_tokens + 15) / 16;
     size_t at = 0;
@@ -514,12 +513,11 @@ static size_t nmoe_sh_layout(size_t max_tokens, uint8_t *base, nmoe_sh_ws *ws) {
     return at;
 }
 
-extern "C" int nmoe_shared_init(nmoe_hip_ctx *ctx) {
+/* Bytes of that scratch; the grouped path's allocation holds it at its end
+ * (one allocation more would lengthen the context's creation). */
+extern "C" size_t nmoe_shared_mm_bytes(int max_tokens) {
     nmoe_sh_ws ws;
-    ctx->s_mm = NULL;
-    if (ctx->max_tokens < NMOE_SHARED_MM_MIN) return NMOE_HIP_OK;
-    return hipMalloc(&ctx->s_mm, nmoe_sh_layout((size_t)ctx->max_tokens, NULL, &ws)) == hipSuccess ? NMOE_HIP_OK
-                                                                                               : NMOE_HIP_ENOMEM;
+    return max_tokens < NMOE_SHARED_MM_MIN ? 0 : nmoe_sh_layout((size_t)max_tokens, NULL, &ws);
 }
 
 template <int PL, int MB, bool GU>
