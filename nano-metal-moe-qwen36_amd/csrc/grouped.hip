@@ -66,7 +66,16 @@ __host__ __device__ constexpr int nmoe_dispatch_blocks(int n) {
     while (nd < NMOE_DISPATCH_MAX && nd * 1024 < n) nd *= 2;
     return nd;
 }
-#define NMOE_MCHUNK 64 /* expert rows (entries) per pass: four 16-row MFMA blocks */
+#define NMOE_MCHUNK 64 /* expert rows (entries) a tile: four 16-row MFMA blocks */
+/* The GEMMs' work list: every expert's entries in pieces of NMOE_MCHUNK, the
+ * last one shorter; so at most one short piece an expert, and whole ones.
+ * This many places (a multiple of 8; those without a piece hold no entries)
+ * cover any routing of n entries, and the GEMM grids are sized for them.  A
+ * block runs one piece: an expert of many entries no longer runs its pieces
+ * one after the other in the blocks of its tiles. */
+__host__ __device__ constexpr int nmoe_work_places(int n) {
+    return (NMOE_EXPERTS + n / NMOE_MCHUNK + 7) / 8 * 8;
+}
 /* Wavefronts per gate/up and down block: 8 (one block a CU) or 4 (two). */
 #ifndef NMOE_GROUPED_NW
 #define NMOE_GROUPED_NW 4
@@ -188,16 +197,14 @@ __device__ __forceinline__ void nmoe_gtl_begin(uint64_t *tl) {
         }
     }
 }
-__device__ __forceinline__ void nmoe_gtl_end(uint64_t *tl, int kind, const uint4 *rank, int es, int nt, int pl,
-                                             int nrows) {
+__device__ __forceinline__ void nmoe_gtl_end(uint64_t *tl, int kind, const uint4 *rank, int es, int nt, int nrows) {
     if constexpr (NMOE_TIMELINE) {
         if (tl != nullptr && threadIdx.x == 0) {
             nmoe_gtl_stamp(tl, NMOE_GTL_END);
             const uint4 rk = rank[es];
             const uint32_t p0 = min(rk.y, (uint32_t)nrows), n = min(rk.z, (uint32_t)nrows - p0);
-            const uint32_t work = n > (uint32_t)(pl * NMOE_MCHUNK) ? n : 0u;
             nmoe_gtl_put(tl, NMOE_GTL_INFO,
-                         ((uint64_t)work << 32) | ((uint64_t)kind << 28) | ((uint64_t)nmoe_xcc_id() << 24) |
+                         ((uint64_t)n << 32) | ((uint64_t)kind << 28) | ((uint64_t)nmoe_xcc_id() << 24) |
                              ((uint64_t)es << 8) | (uint64_t)nt);
         }
     }
@@ -287,11 +294,10 @@ __device__ __forceinline__ void nmoe_dispatch_entries(const nmoe_entry_src &s, i
 
 /* The scatter's LDS counts: per chunk of the first NMOE_DISPATCH_PRE and
  * wavefront, the entries of each expert (then their first places), and
- * the experts' work buckets.  Cleared by nmoe_dispatch_count. */
+ * the short pieces' size classes.  Cleared by nmoe_dispatch_count. */
 struct nmoe_scatter_lds {
     uint32_t wc[NMOE_DISPATCH_PRE][4][NMOE_EXPERTS + 1];
-    uint32_t bk[64];
-    uint32_t wbk[4][64]; /* each wavefront's experts of each work bucket */
+    uint32_t wbk[4][8]; /* each wavefront's short pieces of each size class */
 };
 
 /* D1: h = expert histogram of entry slice b of nd (in LDS). */
@@ -312,13 +318,14 @@ __device__ __forceinline__ void nmoe_dispatch_count(const nmoe_entry_src &s, int
     __syncthreads();
 }
 
-/* The down tiles' order of the one-launch GEMM: order entry es (round
- * g = es / 8 of die d = es mod 8) goes to entry 8 j + d of a second list.
- * A die's large experts (more than NMOE_SMALL_PASS entries, its first nb
+/* The down tiles' order of the one-launch GEMM: work place es (round
+ * g = es / 8 of die d = es mod 8) goes to place 8 j + d of a second list.
+ * A die's large pieces (more than NMOE_SMALL_PASS entries, its first nb
  * rounds) run the longest gate/up tiles, so their down tiles, taken first,
  * would hold their slots waiting; they now come after half of the die's
- * other experts whose gate/up tiles run in the first round of r1 experts
- * (rounds nb .. nb + h - 1 first, then 0 .. nb - 1, then the rest). */
+ * other pieces whose gate/up tiles run in the first round of r1 pieces
+ * (rounds nb .. nb + h - 1 first, then 0 .. nb - 1, then the rest; r1 at most
+ * the list's rounds). */
 __device__ __forceinline__ uint32_t nmoe_down_entry(uint32_t es, uint32_t nbig, uint32_t r1) {
     const uint32_t d = es & 7u, g = es >> 3, r = nbig >> 3, m = nbig & 7u;
     const uint32_t nb = r + (uint32_t)((r & 1u) ? d >= 8u - m : d < m); /* dealt as in the order */
@@ -350,11 +357,11 @@ __device__ __forceinline__ uint32_t nmoe_multisplit9(uint32_t e, int lane, uint3
 template <bool ROUTED, bool MULTI>
 __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src, int ntok, const uint64_t *counts,
                                                       const uint32_t *h, uint32_t *perm, uint32_t *offsets,
-                                                      uint4 *rank, int b, int nd, const uint32_t *ev, uint32_t r1,
-                                                      nmoe_scatter_lds &sl) {
+                                                      uint4 *rank, int ne, int b, int nd, const uint32_t *ev,
+                                                      uint32_t r1, nmoe_scatter_lds &sl) {
     __shared__ uint32_t s_base[NMOE_EXPERTS];
     __shared__ uint32_t s_scan[4]; /* the wavefronts' totals */
-    __shared__ uint32_t s_nbig;    /* the experts of more than one small pass */
+    __shared__ uint32_t s_full[4]; /* and their whole pieces */
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = ntok * src.k;
     const int per = (n + nd - 1) / nd, q0 = b * per, q1 = min(n, (b + 1) * per);
     /* thread e: total of expert e and its count in the slices before b,
@@ -399,23 +406,26 @@ __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src,
          * launch takes the next epoch */
         if (b == 0 && tid == 0) nmoe_add_u32_dev(src.sync + NMOE_SYNC_PREP_EPOCH, 1u);
     }
-    /* the experts by work, most first: bucket = 16-entry row blocks (63 and
-     * more together), a counting sort over the buckets, the experts of one
-     * bucket in index order (any order would do: the GEMM blocks' results
-     * do not depend on it).  The
-     * GEMM blocks take the experts in this order, so the longest tiles start
-     * first and the launch's tail is short.  Entry es runs on die (es + c)
-     * mod 8, so each round of eight is dealt back and forth (0..7, then
-     * 7..0): dealt the same way every round, the same dies would take the
-     * larger expert of every round and finish last. */
-    const int bk = 63 - (int)min((total + 15u) / 16u, 63u);
-    /* (block 0) the expert's place among its wavefront's experts of the same
-     * bucket (a 6-bit multi-split), and each wavefront's count of them */
-    uint32_t brk = 0u;
+    /* the work list, most work first: every expert's whole pieces, then the
+     * short ones by size class (16-entry row blocks, a counting sort), each in
+     * expert order (any order would do: the GEMM blocks' results do not depend
+     * on it).  The GEMM blocks take the pieces in this order, so the longest
+     * tiles start first and the launch's tail is short.  Place es runs on die
+     * (es + c) mod 8, so each round of eight is dealt back and forth (0..7,
+     * then 7..0): dealt the same way every round, the same dies would take the
+     * larger piece of every round and finish last. */
+    const uint32_t full = total / NMOE_MCHUNK, rem = total % NMOE_MCHUNK;
+    static_assert(NMOE_MCHUNK == 64 && NMOE_SMALL_PASS == 16, "size classes 0 .. 3 (three of them large), 4 = none");
+    const int bk = rem != 0u ? 4 - (int)((rem + 15u) / 16u) : 4;
+    /* (block 0) the short piece's place among its wavefront's of the same
+     * class (a 3-bit multi-split), and each wavefront's count of them */
+    uint32_t brk = 0u, finc = 0u;
     if (b == 0) {
         uint32_t bcnt;
-        brk = nmoe_multisplit9<6>((uint32_t)bk, lane, bcnt);
+        brk = nmoe_multisplit9<3>((uint32_t)bk, lane, bcnt);
         if (brk == 0u) sl.wbk[wave][bk] = bcnt;
+        finc = nmoe_wave_incl_scan_u32(full);
+        if (lane == 63) s_full[wave] = finc;
     }
     /* exclusive scan of total over the 256 experts: an inclusive scan within
      * each wavefront (DPP), then the earlier wavefronts' totals */
@@ -454,13 +464,6 @@ __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src,
     if (b == 0) {
         offsets[tid] = off;
         if (tid == 255) offsets[NMOE_EXPERTS] = off + total;
-        if (tid < 64) { /* exclusive scan of the 64 bucket sizes (one wavefront) */
-            const uint32_t c = sl.wbk[0][tid] + sl.wbk[1][tid] + sl.wbk[2][tid] + sl.wbk[3][tid];
-            const uint32_t binc = nmoe_wave_incl_scan_u32(c);
-            sl.bk[tid] = binc - c;
-            static_assert(NMOE_SMALL_PASS == 16, "bucket 62 holds the experts of one small pass");
-            if (tid == 62) s_nbig = binc - c;
-        }
     }
     __syncthreads();
 #pragma unroll
@@ -474,16 +477,35 @@ __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src,
         }
     }
     if (b == 0) {
-        /* the order (its fourth word: the entry itself), and the same
-         * entries in the down tiles' order after it */
-        uint32_t pos = sl.bk[bk] + brk; /* the bucket's first place, the earlier wavefronts', this one's */
+        uint32_t cnt[4], fpos = finc - full, nfull = 0u; /* pieces of each class; the expert's first whole piece */
 #pragma unroll
-        for (int w = 0; w < 3; w++) pos += w < wave ? sl.wbk[w][bk] : 0u;
-        const uint32_t round = pos >> 3;
-        const uint32_t es = 8u * round + ((round & 1u) ? 7u - (pos & 7u) : (pos & 7u));
-        const uint4 ent = make_uint4((uint32_t)tid, off, total, es);
-        rank[es] = ent;
-        rank[NMOE_EXPERTS + nmoe_down_entry(es, s_nbig, r1)] = ent;
+        for (int w = 0; w < 4; w++) {
+            fpos += w < wave ? s_full[w] : 0u;
+            nfull += s_full[w];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) cnt[i] = sl.wbk[0][i] + sl.wbk[1][i] + sl.wbk[2][i] + sl.wbk[3][i];
+        const uint32_t nbig = nfull + cnt[0] + cnt[1] + cnt[2], nwork = nbig + cnt[3], rounds = (uint32_t)ne >> 3;
+        /* the place of position pos (its fourth word: the place itself), and
+         * the same piece in the down tiles' order after it */
+        auto put = [&](uint32_t pos, uint32_t first, uint32_t entries) {
+            if (pos >= (uint32_t)ne) return; /* (counts of a dispatch whose wait gave up) */
+            const uint32_t round = pos >> 3;
+            const uint32_t es = 8u * round + ((round & 1u) ? 7u - (pos & 7u) : (pos & 7u));
+            const uint4 ent = make_uint4((uint32_t)tid, first, entries, es);
+            rank[es] = ent;
+            rank[ne + (int)nmoe_down_entry(es, nbig, min(r1, rounds))] = ent;
+        };
+        for (uint32_t j = 0; j < min(full, (uint32_t)ne); j++) put(fpos + j, off + NMOE_MCHUNK * j, NMOE_MCHUNK);
+        if (rem != 0u) {
+            uint32_t pos = nfull + brk;
+#pragma unroll
+            for (int i = 0; i < 3; i++) pos += i < bk ? cnt[i] : 0u;
+#pragma unroll
+            for (int w = 0; w < 3; w++) pos += w < wave ? sl.wbk[w][bk] : 0u;
+            put(pos, off + NMOE_MCHUNK * full, rem);
+        }
+        for (uint32_t pos = nwork + (uint32_t)tid; pos < (uint32_t)ne; pos += 256u) put(pos, 0u, 0u);
     }
     /* slices of more than NMOE_DISPATCH_PRE chunks: the others one at a
      * time, counted in sl.wc[0] */
@@ -565,9 +587,8 @@ __device__ __forceinline__ void nmoe_grouped_xprep(const XT *x, uint16_t *xhi, u
 static __constant__ uint64_t nmoe_grouped_exp2_tab[32] = NMOE_EXP2_TAB32;
 
 /* The one-launch GEMM's schedule words (zeroed by the preparation launch):
- * done[256], per expert rank, counts the gate/up tiles whose act rows are
+ * done[es], per work place, counts the gate/up tiles whose act rows are
  * stored; each adds 1 + 2^(16 + its die). */
-#define NMOE_SCHED_WORDS NMOE_EXPERTS
 
 /* An expert's done word is touched only by the blocks of one die (its
  * gate/up and down tiles share a die): atomics performed in that die's L2
@@ -622,7 +643,7 @@ __device__ __forceinline__ void nmoe_wait_tiles(uint32_t *cnt, uint32_t n, uint3
 template <int BITS, typename XT, bool ROUTED, bool MULTI>
 __global__ void __launch_bounds__(256) nmoe_grouped_prep_kernel(const uint32_t *idx, int ntok, int k, int nd,
                                                                 uint64_t *counts, uint32_t *perm, uint32_t *offsets,
-                                                                uint4 *rank, uint32_t *sync, uint32_t spin,
+                                                                uint4 *rank, int ne, uint32_t *sync, uint32_t spin,
                                                                 const XT *x, uint16_t *xhi, uint16_t *xlo,
                                                                 uint16_t *xs3, const float *logits, uint32_t *idx_out,
                                                                 float *w_out, uint32_t *done, int skew,
@@ -636,7 +657,7 @@ __global__ void __launch_bounds__(256) nmoe_grouped_prep_kernel(const uint32_t *
      * launch on the stream sees them); rank `skew` (a test of the failure
      * path) from a count no tiles can reach */
     if (done != NULL && b == 0)
-        for (int i = threadIdx.x; i < NMOE_SCHED_WORDS; i += 256) done[i] = i == skew ? 0x8000u : 0u;
+        for (int i = threadIdx.x; i < ne; i += 256) done[i] = i == skew ? 0x8000u : 0u;
     const int nr = ROUTED ? (ntok + 3) / 4 : 0; /* routing blocks */
     if (ROUTED && b >= nd && b < nd + nr) {
         __shared__ float s_sm[4][NMOE_EXPERTS];
@@ -709,11 +730,11 @@ __global__ void __launch_bounds__(256) nmoe_grouped_prep_kernel(const uint32_t *
         for (int i = threadIdx.x; i < NMOE_EXPERTS; i += 256)
             __hip_atomic_store((nmoe_g64 *)&counts[b * NMOE_EXPERTS + i], ((uint64_t)epoch << 32) | h[i],
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    /* experts whose gate/up tiles fill one die's first round: 32 CUs a
+    /* pieces whose gate/up tiles fill one die's first round: 32 CUs a
      * die, two four-wavefront blocks a CU (one of eight) */
     constexpr uint32_t R1 =
         (256u / NMOE_GROUPED_NW) / (uint32_t)(NMOE_INTER / nmoe_gu_rows(sizeof(XT) == 2 ? 1 : 2, NMOE_GROUPED_NW));
-    nmoe_dispatch_scatter<ROUTED, MULTI>(src, ntok, counts, h, perm, offsets, rank, b, nd, ev, R1, s_scat);
+    nmoe_dispatch_scatter<ROUTED, MULTI>(src, ntok, counts, h, perm, offsets, rank, ne, b, nd, ev, R1, s_scat);
     nmoe_gtl_prep_end(tl, 4);
 }
 
@@ -950,23 +971,23 @@ __device__ __forceinline__ void nmoe_wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-/* Block b of a 1-D grid of NMOE_EXPERTS * ntiles blocks -> (expert, tile).
+/* Block b of a 1-D grid of (work places) * ntiles blocks -> (place, tile).
  * Blocks b, b+8, b+16, ... land on the same die (blocks are dealt to the
- * eight dies in turn), so the tiles of one expert run side by side on one
+ * eight dies in turn), so the tiles of one piece run side by side on one
  * die and share its activation rows in that die's L2. */
 __device__ __forceinline__ void nmoe_die_tile(int b, int ntiles, int &e, int &nt) {
     e = 8 * (b / (8 * ntiles)) + (b & 7);
     nt = (b >> 3) % ntiles;
 }
 
-/* Entry es of the expert order (expert, first entry, entries), written by
+/* Place es of the work list (expert, first entry, entries, place), written by
  * the preparation launch and only read by the GEMM launches: one scalar
  * 16-byte load, through the constant address space, all four words needed
  * at once.  Read as a plain pointer, the compiler made it a vector load
  * where it could not prove the words unchanged in the launch (it then
  * waits in the CU's vector memory queue behind the stage loads of the
  * CU's other block) and split it into two dependent loads around the
- * empty-expert exit. */
+ * empty-place exit. */
 __device__ __forceinline__ uint4 nmoe_rank_entry(const uint4 *rank, int es) {
     typedef uint32_t nmoe_v4u __attribute__((ext_vector_type(4)));
     typedef const __attribute__((address_space(4))) nmoe_v4u nmoe_const_v4u;
@@ -1013,12 +1034,11 @@ __host__ __device__ constexpr int nmoe_gu_stages(int bits, int xpl, int nw) {
 }
 
 
-/* Expert e, gate and up rows NT * nt .. +NT-1: act rows of all the
- * expert's entries, 64 entries per pass (16 in one pass in the small
- * form).  NW wavefronts (eight: one block a CU; four: two blocks a CU, whose
+/* A piece of an expert's entries, gate and up rows NT * nt .. +NT-1: the act
+ * rows of its (up to 64; 16 in the small form) entries.  NW wavefronts (eight: one block a CU; four: two blocks a CU, whose
  * set-up and epilogue then overlap the other's ring), two per SIMD either
  * way; wavefront w owns gate and up rows (NT/NW)w .. +NT/NW-1 of the tile as
- * NB 16-row MFMA column blocks each, over the pass's (up to four) 16-entry
+ * NB 16-row MFMA column blocks each, over the piece's (up to four) 16-entry
  * row blocks, so a lane holds gate and up of the same (entry, row).
  *
  * y = sum_g s_g P_g + sum_g (b_g - 128 s_g) xs_g with P_g the MFMA product
@@ -1043,16 +1063,15 @@ struct nmoe_gu_lds_types {
     static_assert(sizeof(StageU) == nmoe_gu_stage_max(BITS, XPL, NW), "stage buffer size");
 };
 
-/* Gate/up tile nt of the es-th expert by entries, pass lane pl, with NS
- * stages in the given LDS buffers (s_st3 is used only with NS = 4).  COUNT:
+/* Gate/up tile nt of work place es, with NS stages in the given LDS buffers (s_st3 is used only with NS = 4).  COUNT:
  * once the tile's act rows and group sums are stored (complete, in this
  * die's L2), the block counts itself in done[es] (nmoe_tile_done), which
  * the down tiles of the same launch wait for. */
 template <int BITS, int XPL, int NW, int NS, bool COUNT>
 __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t *xhi, const uint16_t *xlo,
                                              const uint16_t *xs3, const uint32_t *perm, const uint4 *rank, int k,
-                                             int lanes, int nrows, uint16_t *ahi, uint16_t *alo, float *as, int es,
-                                             int nt, int pl, typename nmoe_gu_lds_types<BITS, XPL, NW>::Scales &s_s,
+                                             int nrows, uint16_t *ahi, uint16_t *alo, float *as, int es, int nt,
+                                             typename nmoe_gu_lds_types<BITS, XPL, NW>::Scales &s_s,
                                              typename nmoe_gu_lds_types<BITS, XPL, NW>::StageU &s_st0,
                                              typename nmoe_gu_lds_types<BITS, XPL, NW>::StageU &s_st1,
                                              typename nmoe_gu_lds_types<BITS, XPL, NW>::StageU &s_st2,
@@ -1073,8 +1092,10 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
      * anything; the clamps keep every access inside the buffers */
     const uint4 rk = nmoe_rank_entry(rank, es);
     const int e = (int)min(rk.x, (uint32_t)(NMOE_EXPERTS - 1));
-    const uint32_t p0 = min(rk.y, (uint32_t)nrows), n = min(rk.z, (uint32_t)nrows - p0);
-    if (n <= (uint32_t)(pl * NMOE_MCHUNK)) return;
+    const uint32_t p0 = min(rk.y, (uint32_t)nrows);
+    uint32_t n = min(min(rk.z, (uint32_t)NMOE_MCHUNK), (uint32_t)nrows - p0);
+    if (n == 0u) return;
+    asm("" : "+s"(n));
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kb = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint8_t *ex = pack + (size_t)e * L::expert_size;
@@ -1087,10 +1108,10 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
     const uint16_t *bias[2] = {(const uint16_t *)(ex + L::gate_b) + (size_t)nt * NT * G,
                                (const uint16_t *)(ex + L::up_b) + (size_t)nt * NT * G};
 
-    /* the passes of one form: MCH entries a pass, GPS groups a ring step */
+    /* the tile in one form: up to MCH entries, GPS groups a ring step */
     auto run = [&](auto mch_c, auto gps_c) {
     constexpr int MCH = decltype(mch_c)::value, GPS = decltype(gps_c)::value;
-    constexpr int MB = MCH / 16;                /* row blocks per full pass */
+    constexpr int MB = MCH / 16;                /* row blocks of a whole piece */
     constexpr int AI = GPS * MCH / 8 / NW;      /* A instructions per plane and wavefront a step */
     static_assert(AI >= 1 && AI * NW * 8 == GPS * MCH, "A rows split evenly over the wavefronts");
     using CR = nmoe_code_row<BITS, GPS>;
@@ -1111,7 +1132,7 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
 #pragma unroll
         for (int b2 = 0; b2 < NB; b2++) coff[u][b2] = nmoe_code_off<BITS, GPS>(rt0 + 16 * b2, u, kb);
 
-    for (uint32_t m0 = pl * MCH; m0 < n; m0 += lanes * MCH) {
+    for (uint32_t m0 = 0; m0 < n; m0 += MCH) { /* once */
         if (tid < MCH) s_tok[tid] = min(perm[p0 + min(m0 + tid, n - 1)], (uint32_t)nrows - 1u) / (uint32_t)k;
         nmoe_lds_barrier();
         /* this lane's A row for instruction j = wave + NW i (rows 8j .. 8j+7
@@ -1148,8 +1169,8 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
              * LDS read of the scales). */
             constexpr int PER = 2 * NT * G / 8 / NTH;
             static_assert(PER * NTH == 2 * NT * G / 8, "scale chunks split evenly over the threads");
-            /* the tile's scales straight into LDS, every pass (later
-             * passes hit L2): wavefront w's q-th 1 KB at uint4 NTH q + 64w */
+            /* the tile's scales straight into LDS: wavefront w's q-th 1 KB
+             * at uint4 NTH q + 64w */
 #pragma unroll
             for (int q = 0; q < PER; q++) {
                 /* LDS chunk i = (mat, chunk, row) <- global chunk row * G/8 + chunk of the matrix */
@@ -1312,10 +1333,9 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
             for (int q = 1; q < WPD; q++) t = t + s_as[WPD * dg + q][row];
             if (m < n) as[(size_t)(p0 + m) * (NMOE_INTER / NMOE_GROUP) + DG * nt + dg] = t;
         }
-        nmoe_lds_barrier(); /* s_tok, s_as and the stages are reused by the next pass */
     }
     };
-    /* block-uniform: the expert's entry count picks the form */
+    /* block-uniform: the piece's entry count picks the form */
     if constexpr (nmoe_small_form(NW)) {
         if (n <= (uint32_t)NMOE_SMALL_PASS)
             run(std::integral_constant<int, NMOE_SMALL_PASS>{}, std::integral_constant<int, NMOE_SMALL_GPS>{});
@@ -1336,26 +1356,22 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
 template <int BITS, int XPL, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 nmoe_grouped_gateup_kernel(const uint8_t *pack, const uint16_t *xhi, const uint16_t *xlo, const uint16_t *xs3,
-                           const uint32_t *perm, const uint4 *rank, int k, int lanes, int nrows, uint16_t *ahi,
-                           uint16_t *alo, float *as, uint64_t *tl) {
+                           const uint32_t *perm, const uint4 *rank, int k, int nrows, uint16_t *ahi, uint16_t *alo,
+                           float *as, uint64_t *tl) {
     nmoe_gtl_begin(tl);
     typedef nmoe_gu_lds_types<BITS, XPL, NW> T;
     __shared__ typename T::Scales s_s;
     __shared__ typename T::StageU s_st0, s_st1, s_st2, s_st3;
     __shared__ uint32_t s_tok[NMOE_MCHUNK];
     __shared__ float s_as[NW][NMOE_MCHUNK];
-    /* pass lane pl of `lanes`: passes pl, pl + lanes, ... of tile (e, nt);
-     * the tile's expert is the es-th by entries (most first), so the
-     * longest tiles start first */
     constexpr int NTILE = NMOE_INTER / T::NT;
-    const int pl = blockIdx.x / (NMOE_EXPERTS * NTILE);
     int es, nt;
-    nmoe_die_tile(blockIdx.x % (NMOE_EXPERTS * NTILE), NTILE, es, nt);
+    nmoe_die_tile(blockIdx.x, NTILE, es, nt);
     /* (five stages measured no faster than four) */
-    nmoe_gu_tile<BITS, XPL, NW, nmoe_gu_stages(BITS, XPL, NW), false>(pack, xhi, xlo, xs3, perm, rank, k, lanes, nrows,
-                                                                      ahi, alo, as, es, nt, pl, s_s, s_st0, s_st1,
-                                                                      s_st2, s_st3, s_tok, s_as, NULL);
-    nmoe_gtl_end(tl, 1, rank, es, nt, pl, nrows);
+    nmoe_gu_tile<BITS, XPL, NW, nmoe_gu_stages(BITS, XPL, NW), false>(pack, xhi, xlo, xs3, perm, rank, k, nrows, ahi,
+                                                                      alo, as, es, nt, s_s, s_st0, s_st1, s_st2,
+                                                                      s_st3, s_tok, s_as, NULL);
+    nmoe_gtl_end(tl, 1, rank, es, nt, nrows);
 }
 
 /* ------------------------------------------------------------ down */
@@ -1395,16 +1411,15 @@ struct nmoe_dn_lds_types {
     static_assert(sizeof(StageU) == nmoe_dn_stage_max(BITS, NW, NT), "stage buffer size");
 };
 
-/* Down tile nt (NT rows) of the es-th expert by entries, pass lane pl:
- * y[q][row] for all the expert's entries q, 64 per pass (16 in one pass in
- * the small form), with NS stages in the given LDS buffers.  NW wavefronts
+/* Down tile nt (NT rows) of work place es: y[q][row] for the piece's entries
+ * q, with NS stages in the given LDS buffers.  NW wavefronts
  * (as in the gate/up kernel); wavefront w owns rows (NT/NW)w .. +NT/NW-1 of
  * the tile as NB 16-row column blocks.  act enters as hi and lo bf16
  * planes.
  *
  * WAIT (the gate/up tiles run in the same launch): with its weight loads
- * in flight, a bounded wait until done[es] counts all gu_tiles gate/up
- * tiles of each pass lane that has work; those ran on this block's die (the
+ * in flight, a bounded wait until done[] counts the piece's gu_tiles gate/up
+ * tiles; those ran on this block's die (the
  * same block index mod 8; nmoe_wait_tiles checks it), so their act rows
  * are in this die's L2.  The act rows are then read through L1 as usual (no
  * block of this launch read them before they were complete: an act row is
@@ -1412,14 +1427,14 @@ struct nmoe_dn_lds_types {
  * lines with other experts' rows, with loads that bypass L1. */
 template <int BITS, int NW, int NT, int NS, bool WAIT>
 __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t *ahi, const uint16_t *alo,
-                                             const float *as, const uint32_t *perm, const uint4 *rank, int lanes,
-                                             int nrows, float *y, int es, int nt, int pl,
+                                             const float *as, const uint32_t *perm, const uint4 *rank, int nrows,
+                                             float *y, int es, int nt,
                                              typename nmoe_dn_lds_types<BITS, NW, NT>::Scales &s_s,
                                              typename nmoe_dn_lds_types<BITS, NW, NT>::StageU &s_st0,
                                              typename nmoe_dn_lds_types<BITS, NW, NT>::StageU &s_st1,
                                              typename nmoe_dn_lds_types<BITS, NW, NT>::StageU &s_st2,
                                              typename nmoe_dn_lds_types<BITS, NW, NT>::StageU &s_st3,
-                                             uint32_t (&s_q)[NMOE_MCHUNK], uint32_t *done, int gu_tiles,
+                                             uint32_t (&s_q)[NMOE_MCHUNK], uint32_t *done, int ne, int gu_tiles,
                                              uint32_t *sync, uint32_t spin, uint64_t *tl) {
     using Q = nmoe_q<BITS>;
     using L = nmoe_layout<BITS>;
@@ -1432,8 +1447,10 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     typedef typename nmoe_dn_lds_types<BITS, NW, NT>::StageU StageU;
     const uint4 rk = nmoe_rank_entry(rank, es); /* clamped as in the gate/up kernel */
     const int e = (int)min(rk.x, (uint32_t)(NMOE_EXPERTS - 1));
-    const uint32_t p0 = min(rk.y, (uint32_t)nrows), n = min(rk.z, (uint32_t)nrows - p0);
-    if (n <= (uint32_t)(pl * NMOE_MCHUNK)) return;
+    const uint32_t p0 = min(rk.y, (uint32_t)nrows);
+    uint32_t n = min(min(rk.z, (uint32_t)NMOE_MCHUNK), (uint32_t)nrows - p0);
+    if (n == 0u) return;
+    asm("" : "+s"(n));
     static_assert(!WAIT || NS == 3, "the split prologue's waits are written for three stages");
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kb = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1442,10 +1459,10 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     const uint32_t *cbase = (const uint32_t *)(ex + L::down_w); /* stripe-major */
     const uint16_t *bias = (const uint16_t *)(ex + L::down_b) + (size_t)nt * NT * G;
 
-    /* the passes of one form: MCH entries a pass, GPS groups a ring step */
+    /* the tile in one form: up to MCH entries, GPS groups a ring step */
     auto run = [&](auto mch_c, auto gps_c) {
     constexpr int MCH = decltype(mch_c)::value, GPS = decltype(gps_c)::value;
-    constexpr int MB = MCH / 16;           /* row blocks per full pass */
+    constexpr int MB = MCH / 16;           /* row blocks of a whole piece */
     constexpr int AI = GPS * MCH / 8 / NW; /* A instructions per plane and wavefront a step */
     static_assert(AI >= 1 && AI * NW * 8 == GPS * MCH, "A rows split evenly over the wavefronts");
     using CR = nmoe_code_row<BITS, GPS>;
@@ -1462,13 +1479,13 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     for (int u = 0; u < GPS; u++)
 #pragma unroll
         for (int b2 = 0; b2 < NB; b2++) coff[u][b2] = nmoe_code_off<BITS, GPS>(rt0 + 16 * b2, u, kb);
-    for (uint32_t m0 = pl * MCH; m0 < n; m0 += lanes * MCH) {
+    for (uint32_t m0 = 0; m0 < n; m0 += MCH) { /* once */
         /* the chunk's output slots, stored to LDS after the stages are issued
          * (so that this load's wait does not hold them back) and visible
          * after the barrier below */
         const uint32_t qv = tid < MCH ? min(perm[p0 + min(m0 + tid, n - 1)], (uint32_t)nrows - 1u) : 0u;
         /* this lane's A row for instruction j = wave + NW i (group
-         * j / (MCH / 8) of the step): act row p0 + m0 + 8 (j % (MCH / 8)) +
+         * j / (MCH / 8) of the step): act row p0 + 8 (j % (MCH / 8)) +
          * lane / 8 */
         uint32_t row_off[AI];
 #pragma unroll
@@ -1500,8 +1517,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
         nmoe_f32x4 acc[NB][MB];
         {
             /* as in the gate/up kernel: the correction's operands
-             * (scales straight into LDS, one 16-byte chunk a thread,
-             * every pass), then the first ring stages, then a wait that
+             * (scales straight into LDS, one 16-byte chunk a thread), then the first ring stages, then a wait that
              * leaves only the stages in flight.
              * A lane = (entry col, groups 2kb + tq), B lane = (row col,
              * groups 2kb + tq) */
@@ -1525,8 +1541,8 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
             };
             if constexpr (WAIT) {
                 /* the weights first (they do not wait for the gate/up
-                 * tiles): biases and the first stages' codes; then, on the
-                 * first pass, the wait for the expert's gate/up tiles (a
+                 * tiles): biases and the first stages' codes; then the wait
+                 * for the piece's gate/up tiles (a
                  * barrier that leaves the loads in flight); then the act
                  * side: group sums and the first stages' act rows.  The wait
                  * below leaves only stage 1's act rows in flight, so stage 0
@@ -1535,15 +1551,12 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
                 for (int b2 = 0; b2 < NB; b2++) bv[b2] = *(const uint32_t *)(bias + (rt0 + 16 * b2) * G + 2 * kb);
 #pragma unroll
                 for (int st = 0; st < NS - 1; st++) issue_b(st, st);
-                if (m0 == (uint32_t)(pl * MCH)) {
-                    if (tid == 0) {
-                        const uint32_t busy = min((uint32_t)lanes, (n + NMOE_MCHUNK - 1) / NMOE_MCHUNK);
-                        /* the entry's fourth word: its place in the gate/up order */
-                        nmoe_wait_tiles(done + (rk.w & (NMOE_EXPERTS - 1)), (uint32_t)gu_tiles * busy, sync, spin);
-                        nmoe_gtl_stamp(tl, NMOE_GTL_READY);
-                    }
-                    nmoe_lds_barrier();
+                if (tid == 0) {
+                    /* the fourth word: the piece's place in the gate/up order */
+                    nmoe_wait_tiles(done + min(rk.w, (uint32_t)ne - 1u), (uint32_t)gu_tiles, sync, spin);
+                    nmoe_gtl_stamp(tl, NMOE_GTL_READY);
                 }
+                nmoe_lds_barrier();
                 load_av();
 #pragma unroll
                 for (int st = 0; st < NS - 1; st++) issue_a(st, st);
@@ -1633,11 +1646,10 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
                 }
             }
         }
-        nmoe_lds_barrier(); /* the stages and s_q are reused by the next pass */
     }
     };
-    /* block-uniform: the expert's entry count picks the form */
-    if constexpr (nmoe_small_form(NW)) {
+    /* block-uniform: the piece's entry count picks the form */
+    if constexpr (nmoe_small_form(NW) && WAIT) {
         if (n <= (uint32_t)NMOE_SMALL_PASS) {
             run(std::integral_constant<int, NMOE_SMALL_PASS>{}, std::integral_constant<int, NMOE_SMALL_GPS>{});
             return;
@@ -1649,22 +1661,20 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
 template <int BITS, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 nmoe_grouped_down_kernel(const uint8_t *pack, const uint16_t *ahi, const uint16_t *alo, const float *as,
-                         const uint32_t *perm, const uint4 *rank, int lanes, int nrows, float *y, uint64_t *tl) {
+                         const uint32_t *perm, const uint4 *rank, int nrows, float *y, uint64_t *tl) {
     nmoe_gtl_begin(tl);
     constexpr int NT = nmoe_dn_rows(NW);
     typedef nmoe_dn_lds_types<BITS, NW, NT> T;
     __shared__ typename T::Scales s_s;
     __shared__ typename T::StageU s_st0, s_st1, s_st2, s_st3;
     __shared__ uint32_t s_q[NMOE_MCHUNK]; /* the chunk's output slots */
-    /* pass lane and tile as in the gate/up kernel */
     constexpr int NTILE = NMOE_HIDDEN / NT;
-    const int pl = blockIdx.x / (NMOE_EXPERTS * NTILE);
     int es, nt;
-    nmoe_die_tile(blockIdx.x % (NMOE_EXPERTS * NTILE), NTILE, es, nt);
-    nmoe_dn_tile<BITS, NW, NT, nmoe_dn_stages(BITS, NW), false>(pack, ahi, alo, as, perm, rank, lanes, nrows, y, es,
-                                                                nt, pl, s_s, s_st0, s_st1, s_st2, s_st3, s_q, NULL, 0,
-                                                                NULL, 0u, NULL);
-    nmoe_gtl_end(tl, 2, rank, es, nt, pl, nrows);
+    nmoe_die_tile(blockIdx.x, NTILE, es, nt);
+    nmoe_dn_tile<BITS, NW, NT, nmoe_dn_stages(BITS, NW), false>(pack, ahi, alo, as, perm, rank, nrows, y, es, nt, s_s,
+                                                                s_st0, s_st1, s_st2, s_st3, s_q, NULL, 0, 0, NULL, 0u,
+                                                                NULL);
+    nmoe_gtl_end(tl, 2, rank, es, nt, nrows);
 }
 
 /* ------------------------------------------------------------ gate/up + down in one launch */
@@ -1684,21 +1694,20 @@ __host__ __device__ constexpr int nmoe_ffn_lds(int bits, int xpl, int nw, int ns
  * blocks have no room for a fourth; eight-wavefront ones take three too). */
 __host__ __device__ constexpr int nmoe_ffn_stages(int, int, int) { return 3; }
 
-/* Gate/up and down of the grouped experts in one launch (one pass lane):
- * blocks 0 .. ngu-1 are the gate/up tiles (as nmoe_grouped_gateup_kernel's
+/* Gate/up and down of the grouped experts in one launch: blocks 0 .. ngu-1 are the gate/up tiles (as nmoe_grouped_gateup_kernel's
  * grid), the blocks after them the down tiles of nmoe_ffn_dn_rows(NW) rows
  * (as nmoe_grouped_down_kernel's grid, from block ngu on, over the second
  * list of rank[]: the down tiles' order, nmoe_down_entry).  A down tile
- * waits (bounded) for its expert's gate/up tiles, which count themselves in
- * done[] (zeroed by the preparation launch) at the expert's gate/up entry,
- * so the down tiles of the experts finished first fill the CUs that the
+ * waits (bounded) for its piece's gate/up tiles, which count themselves in
+ * done[] (zeroed by the preparation launch) at the piece's gate/up place,
+ * so the down tiles of the pieces finished first fill the CUs that the
  * last gate/up tiles leave idle, instead of waiting for the whole gate/up
  * launch to end.
  *
  * Where the tiles run: blocks are dealt to the eight dies in turn, block b
  * to die (b + c) mod 8 with c fixed within the launch (checked at context
  * creation, else this kernel is not used), and ngu is a multiple of 8, so
- * the gate/up and down tiles of one expert (the same entry mod 8 in either
+ * the gate/up and down tiles of one piece (the same place mod 8 in either
  * order) run on one die and its L2 holds their act rows (nmoe_wait_tiles
  * checks it).
  * A die starts its blocks in index order, so every gate/up block a down
@@ -1707,8 +1716,8 @@ __host__ __device__ constexpr int nmoe_ffn_stages(int, int, int) { return 3; }
 template <int BITS, int XPL, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 nmoe_grouped_ffn_kernel(const uint8_t *pack, const uint16_t *xhi, const uint16_t *xlo, const uint16_t *xs3,
-                        const uint32_t *perm, const uint4 *rank, int k, int nrows, uint16_t *ahi, uint16_t *alo,
-                        float *as, float *y, int ngu, uint32_t *done, uint32_t *sync, uint32_t spin, uint64_t *tl) {
+                        const uint32_t *perm, const uint4 *rank, int ne, int k, int nrows, uint16_t *ahi,
+                        uint16_t *alo, float *as, float *y, int ngu, uint32_t *done, uint32_t *sync, uint32_t spin, uint64_t *tl) {
     nmoe_gtl_begin(tl);
     typedef nmoe_gu_lds_types<BITS, XPL, NW> TG;
     constexpr int NTD = nmoe_ffn_dn_rows(NW);
@@ -1733,16 +1742,16 @@ nmoe_grouped_ffn_kernel(const uint8_t *pack, const uint16_t *xhi, const uint16_t
     int es, nt;
     if ((int)blockIdx.x < ngu) {
         nmoe_die_tile(blockIdx.x, NTG, es, nt);
-        nmoe_gu_tile<BITS, XPL, NW, NS, true>(pack, xhi, xlo, xs3, perm, rank, k, 1, nrows, ahi, alo, as, es, nt, 0,
+        nmoe_gu_tile<BITS, XPL, NW, NS, true>(pack, xhi, xlo, xs3, perm, rank, k, nrows, ahi, alo, as, es, nt,
                                               s_s.gu, s_st0.gu, s_st1.gu, s_st2.gu, s_st3.gu, s_tok, s_as, done);
-        nmoe_gtl_end(tl, 1, rank, es, nt, 0, nrows);
+        nmoe_gtl_end(tl, 1, rank, es, nt, nrows);
     } else {
         /* the down tiles' order (the dispatch's second list) */
         nmoe_die_tile(blockIdx.x - ngu, NTILED, es, nt);
-        nmoe_dn_tile<BITS, NW, NTD, NS, true>(pack, ahi, alo, as, perm, rank + NMOE_EXPERTS, 1, nrows, y, es, nt, 0,
-                                              s_s.dn, s_st0.dn, s_st1.dn, s_st2.dn, s_st3.dn, s_tok, done, NTG, sync,
-                                              spin, tl);
-        nmoe_gtl_end(tl, 2, rank + NMOE_EXPERTS, es, nt, 0, nrows);
+        nmoe_dn_tile<BITS, NW, NTD, NS, true>(pack, ahi, alo, as, perm, rank + ne, nrows, y, es, nt, s_s.dn,
+                                              s_st0.dn, s_st1.dn, s_st2.dn, s_st3.dn, s_tok, done, ne, NTG, sync, spin,
+                                              tl);
+        nmoe_gtl_end(tl, 2, rank + ne, es, nt, nrows);
     }
 }
 
@@ -1862,13 +1871,13 @@ int nmoe_pack_stripe(nmoe_hip_ctx *ctx, int layer) {
 extern "C" size_t nmoe_shared_mm_bytes(int max_tokens);
 
 extern "C" int nmoe_grouped_init(nmoe_hip_ctx *ctx) {
-    const size_t mt = (size_t)ctx->max_tokens, rows = mt * NMOE_MAX_K;
+    const size_t mt = (size_t)ctx->max_tokens, rows = mt * NMOE_MAX_K, places = (size_t)nmoe_work_places((int)rows);
     const size_t y_bytes = rows * NMOE_HIDDEN * sizeof(float), mm_bytes = nmoe_shared_mm_bytes(ctx->max_tokens);
     ctx->grouped_min_tokens = 8;
     if (hipMalloc((void **)&ctx->g_counts, NMOE_DISPATCH_MAX * NMOE_EXPERTS * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_perm, rows * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_offsets, (NMOE_EXPERTS + 1) * sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc((void **)&ctx->g_rank, 2 * NMOE_EXPERTS * 4 * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc((void **)&ctx->g_rank, 2 * places * 4 * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_xhi, mt * NMOE_HIDDEN * sizeof(uint16_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_xlo, mt * NMOE_HIDDEN * sizeof(uint16_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_xs, mt * 3 * (NMOE_HIDDEN / NMOE_GROUP) * sizeof(uint16_t)) != hipSuccess ||
@@ -1876,7 +1885,7 @@ extern "C" int nmoe_grouped_init(nmoe_hip_ctx *ctx) {
         hipMalloc((void **)&ctx->g_alo, rows * NMOE_INTER * sizeof(uint16_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_as, rows * (NMOE_INTER / NMOE_GROUP) * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_y, y_bytes + mm_bytes) != hipSuccess ||
-        hipMalloc((void **)&ctx->g_done, NMOE_SCHED_WORDS * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc((void **)&ctx->g_done, places * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_tags, rows * sizeof(uint64_t)) != hipSuccess)
         return NMOE_HIP_ENOMEM;
     ctx->s_mm = mm_bytes != 0 ? (uint8_t *)ctx->g_y + y_bytes : NULL; /* (y_bytes is a multiple of 64 KB) */
@@ -1888,8 +1897,8 @@ extern "C" int nmoe_grouped_init(nmoe_hip_ctx *ctx) {
     if (hipMemset(ctx->g_counts, 0, NMOE_DISPATCH_MAX * NMOE_EXPERTS * sizeof(uint64_t)) != hipSuccess ||
         hipMemset(ctx->g_perm, 0, rows * sizeof(uint32_t)) != hipSuccess ||
         hipMemset(ctx->g_offsets, 0, (NMOE_EXPERTS + 1) * sizeof(uint32_t)) != hipSuccess ||
-        hipMemset(ctx->g_rank, 0, 2 * NMOE_EXPERTS * 4 * sizeof(uint32_t)) != hipSuccess ||
-        hipMemset(ctx->g_done, 0, NMOE_SCHED_WORDS * sizeof(uint32_t)) != hipSuccess ||
+        hipMemset(ctx->g_rank, 0, 2 * places * 4 * sizeof(uint32_t)) != hipSuccess ||
+        hipMemset(ctx->g_done, 0, places * sizeof(uint32_t)) != hipSuccess ||
         hipMemset(ctx->g_tags, 0, rows * sizeof(uint64_t)) != hipSuccess ||
         hipDeviceSynchronize() != hipSuccess)
         return NMOE_HIP_EHIP;
@@ -1909,7 +1918,8 @@ extern "C" int nmoe_grouped_dispatch(nmoe_hip_ctx *ctx, const uint32_t *idx, int
     const int nd = nmoe_dispatch_blocks(ntok * k);
 #define NMOE_DISPATCH_LAUNCH(M)                                                                                        \
     hipLaunchKernelGGL((nmoe_grouped_prep_kernel<4, uint16_t, false, M>), dim3(nd), dim3(256), 0, s, idx, ntok, k, nd, \
-                       ctx->g_counts, perm, offsets, (uint4 *)ctx->g_rank, ctx->sync, ctx->spin_limit,                 \
+                       ctx->g_counts, perm, offsets, (uint4 *)ctx->g_rank, nmoe_work_places(ntok * k), ctx->sync,      \
+                       ctx->spin_limit,                                                                                \
                        (const uint16_t *)NULL, (uint16_t *)NULL, (uint16_t *)NULL, (uint16_t *)NULL,                   \
                        (const float *)NULL, (uint32_t *)NULL, (float *)NULL, (uint32_t *)NULL, -1, (uint64_t *)NULL,    \
                        (uint64_t *)NULL)
@@ -1933,13 +1943,11 @@ static int nmoe_grouped_run(nmoe_hip_ctx *ctx, const uint8_t *pack, const void *
     const dim3 gprep(nd + (logits != NULL ? (ntok + 3) / 4 : 0) + ntok);
     uint32_t *ri = (uint32_t *)idx;
     float *rw = (float *)w;
-    /* two pass lanes once an expert averages more than half a pass: the
-     * passes of a large expert's tile then run in blocks of their own, side
-     * by side (on the same die, so the second reads the codes from L2) */
-    const int lanes = (long)ntok * k > (long)NMOE_EXPERTS * NMOE_MCHUNK / 2 ? 2 : 1;
-    /* gate/up and down in one launch where the blocks' dies are known (one
-     * pass lane) */
-    const bool one = ctx->grouped_one_launch && ctx->xcd_placed && lanes == 1;
+    const int ne = nmoe_work_places(ntok * k);
+    /* gate/up and down in one launch where the blocks' dies are known, up to
+     * 32 entries an expert on average; beyond, the one-launch form's smaller
+     * down tiles cost more than the overlap gains */
+    const bool one = ctx->grouped_one_launch && ctx->xcd_placed && (long)ntok * k <= (long)NMOE_EXPERTS * NMOE_MCHUNK / 2;
     uint32_t *done = one ? ctx->g_done : NULL;
     const int skew = one ? ctx->skew_tiles : -1;
     if (one) ctx->skew_tiles = -1;
@@ -1947,7 +1955,7 @@ static int nmoe_grouped_run(nmoe_hip_ctx *ctx, const uint8_t *pack, const void *
     uint64_t *tlp = nmoe_tl_take(ctx, (int)((4 * (size_t)gprep.x + NMOE_TL_SLOT_WORDS - 1) / NMOE_TL_SLOT_WORDS));
 #define NMOE_PREP_M(XT, R, XLO, M)                                                                                      \
     hipLaunchKernelGGL((nmoe_grouped_prep_kernel<BITS, XT, R, M>), gprep, dim3(256), 0, s, idx, ntok, k, nd,              \
-                       ctx->g_counts, ctx->g_perm, ctx->g_offsets, (uint4 *)ctx->g_rank, ctx->sync, ctx->spin_limit,    \
+                       ctx->g_counts, ctx->g_perm, ctx->g_offsets, (uint4 *)ctx->g_rank, ne, ctx->sync, ctx->spin_limit, \
                        (const XT *)x, ctx->g_xhi, XLO, ctx->g_xs, logits, ri, rw, done, skew, ctx->g_tags, tlp)
     /* (one slice: the form without the slices' histogram exchange, and its registers) */
 #define NMOE_PREP(XT, R, XLO)                 \
@@ -1972,8 +1980,7 @@ static int nmoe_grouped_run(nmoe_hip_ctx *ctx, const uint8_t *pack, const void *
 #undef NMOE_PREP_M
     constexpr int NW = NMOE_GROUPED_NW;
     const dim3 blk(64 * NW);
-    const dim3 ggu(lanes * NMOE_EXPERTS * (NMOE_INTER / nmoe_gu_rows(bf ? 1 : 2, NW))),
-        gdn(lanes * NMOE_EXPERTS * (NMOE_HIDDEN / nmoe_dn_rows(NW)));
+    const dim3 ggu(ne * (NMOE_INTER / nmoe_gu_rows(bf ? 1 : 2, NW))), gdn(ne * (NMOE_HIDDEN / nmoe_dn_rows(NW)));
     const uint16_t *xhi = (const uint16_t *)ctx->g_xhi, *xlo = (const uint16_t *)ctx->g_xlo;
     const uint32_t *perm = (const uint32_t *)ctx->g_perm;
     const uint4 *rank = (const uint4 *)ctx->g_rank;
@@ -1982,7 +1989,7 @@ static int nmoe_grouped_run(nmoe_hip_ctx *ctx, const uint8_t *pack, const void *
     const float *as = (const float *)ctx->g_as;
     const int nrows = ntok * k;
     /* timeline builds: 4 stamps a block of the GEMM launches */
-    const dim3 gffn(ggu.x + NMOE_EXPERTS * (NMOE_HIDDEN / nmoe_ffn_dn_rows(NW)));
+    const dim3 gffn(ggu.x + ne * (NMOE_HIDDEN / nmoe_ffn_dn_rows(NW)));
     const size_t tl_recs = one ? gffn.x : ggu.x + gdn.x;
     const int tl_slots = (int)((4 * tl_recs + NMOE_TL_SLOT_WORDS - 1) / NMOE_TL_SLOT_WORDS);
     uint64_t *tl = nmoe_tl_take(ctx, tl_slots);
@@ -1990,22 +1997,22 @@ static int nmoe_grouped_run(nmoe_hip_ctx *ctx, const uint8_t *pack, const void *
         /* gate/up tiles, then the down tiles of nmoe_ffn_dn_rows rows, in one grid */
         if (bf)
             hipLaunchKernelGGL((nmoe_grouped_ffn_kernel<BITS, 1, NW>), gffn, blk, 0, s, pack, xhi, xlo, xs3, perm, rank,
-                               k, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, ctx->g_y, (int)ggu.x, done, ctx->sync,
+                               ne, k, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, ctx->g_y, (int)ggu.x, done, ctx->sync,
                                ctx->spin_limit, tl);
         else
             hipLaunchKernelGGL((nmoe_grouped_ffn_kernel<BITS, 2, NW>), gffn, blk, 0, s, pack, xhi, xlo, xs3, perm, rank,
-                               k, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, ctx->g_y, (int)ggu.x, done, ctx->sync,
+                               ne, k, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, ctx->g_y, (int)ggu.x, done, ctx->sync,
                                ctx->spin_limit, tl);
     } else {
         /* gate/up, then down */
         if (bf)
             hipLaunchKernelGGL((nmoe_grouped_gateup_kernel<BITS, 1, NW>), ggu, blk, 0, s, pack, xhi, xlo, xs3, perm,
-                               rank, k, lanes, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, tl);
+                               rank, k, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, tl);
         else
             hipLaunchKernelGGL((nmoe_grouped_gateup_kernel<BITS, 2, NW>), ggu, blk, 0, s, pack, xhi, xlo, xs3, perm,
-                               rank, k, lanes, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, tl);
-        hipLaunchKernelGGL((nmoe_grouped_down_kernel<BITS, NW>), gdn, blk, 0, s, pack, ahi, alo, as, perm, rank, lanes,
-                           nrows, ctx->g_y, tl == NULL ? tl : tl + 4 * (size_t)ggu.x);
+                               rank, k, nrows, ctx->g_ahi, ctx->g_alo, ctx->g_as, tl);
+        hipLaunchKernelGGL((nmoe_grouped_down_kernel<BITS, NW>), gdn, blk, 0, s, pack, ahi, alo, as, perm, rank, nrows,
+                           ctx->g_y, tl == NULL ? tl : tl + 4 * (size_t)ggu.x);
     }
     const uint32_t *status = ctx->sync + NMOE_SYNC_STATUS;
     if (nmoe_aligned(h_mid, 16) && nmoe_aligned(out, 16) && (shared_out == NULL || nmoe_aligned(shared_out, 16)))

@@ -123,13 +123,13 @@ struct nmoe_hip_ctx {
     int grouped_min_tokens; /* NMOE_HIP_OPT_GROUPED_MIN_TOKENS */
     int grouped_one_launch; /* NMOE_HIP_OPT_GROUPED_ONE_LAUNCH */
     int skew_tiles;         /* NMOE_HIP_OPT_SKEW_TILES: rank, or -1 */
-    uint32_t *g_done;       /* [256] the one-launch form's gate/up tiles done per expert rank */
+    uint32_t *g_done;       /* [places] the one-launch form's gate/up tiles done per work place */
     uint64_t *g_tags;       /* [T*8] routed entries of the preparation launch: epoch << 32 | expert */
     uint64_t *g_counts;     /* [64][256] per-slice expert histograms, each word epoch << 32 | count */
     uint32_t *g_perm;       /* [T*8] entries grouped by expert */
     uint32_t *g_offsets;    /* [257] */
-    uint32_t *g_rank;       /* [2][256][4] the expert order (expert, first entry, entries, entry), then the
-                               same entries in the one-launch down tiles' order */
+    uint32_t *g_rank;       /* [2][places][4] the work list (expert, first entry, entries, place), then the
+                               same pieces in the one-launch down tiles' order */
     uint16_t *g_xhi, *g_xlo; /* [T][2048] x in operand order (bf16 hi / lo) */
     uint16_t *g_xs;         /* [T][3][32] group sums of x as three bf16 parts */
     uint16_t *g_ahi, *g_alo; /* [T*8][512] act (bf16 hi / lo), by permuted row */
