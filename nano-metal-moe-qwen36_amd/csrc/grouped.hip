@@ -770,26 +770,26 @@ union nmoe_stage_buf {
     S small;
 };
 
-/* A direct load into LDS from a wavefront-uniform base plus a 32-bit
- * per-lane byte offset: the compiler can address it as a scalar base and a
- * vector offset, so the stages' per-group addresses cost no vector
- * registers (the group moves the scalar base). */
+/* A direct load into LDS through a buffer resource: the lane's constant byte
+ * offset in a vector register, the group's in a scalar one, so a stage's
+ * loads cost no vector instructions (as global loads they took a 64-bit
+ * address addition each, ten or more of a step's 140 vector instructions,
+ * and those bound the ring). */
 template <int SZ>
-__device__ __forceinline__ void nmoe_dma(const void *ubase, uint32_t off, void *lds) {
-    const void *src = (const void *)((const char *)ubase + off);
+__device__ __forceinline__ void nmoe_dma(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, void *lds) {
     if constexpr (SZ == 16)
-        __builtin_amdgcn_global_load_lds(src, (nmoe_lds_void *)lds, 16, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (nmoe_lds_void *)lds, 16, (int)voff, (int)soff, 0, 0);
     else
-        __builtin_amdgcn_global_load_lds(src, (nmoe_lds_void *)lds, 4, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (nmoe_lds_void *)lds, 4, (int)voff, (int)soff, 0, 0);
 }
 
-/* Instruction j (rows 8j..8j+7) of one A plane: ubase is the plane at the
- * group's first column (uniform), row_off this lane's row (8j + lane / 8)
- * in bytes. */
-__device__ __forceinline__ void nmoe_stage_rows(uint4 *plane, const uint16_t *ubase, uint32_t row_off, int j, int lane) {
+/* Instruction j (rows 8j..8j+7) of one A plane (buffer pr): group `group`'s
+ * columns (uniform), row_off this lane's row (8j + lane / 8) in bytes. */
+__device__ __forceinline__ void nmoe_stage_rows(uint4 *plane, __amdgpu_buffer_rsrc_t pr, int group, uint32_t row_off,
+                                                int j, int lane) {
     const int r = 8 * j + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
-    nmoe_dma<16>(ubase, row_off + 16u * (uint32_t)c, plane + 64 * j);
+    nmoe_dma<16>(pr, row_off + 16u * (uint32_t)c, 128u * (uint32_t)group, plane + 64 * j);
 }
 
 /* MFMA A operand (the lane's two 8-element chunks 2kb, 2kb+1) of row r. */
@@ -845,24 +845,24 @@ __host__ __device__ __forceinline__ uint32_t nmoe_stripe_word(uint32_t r, uint32
 }
 
 /* Instruction j of one stage's codes for rows row0 .. row0 + NR - 1 of a
- * stripe-major matrix at mbase, groups
+ * stripe-major matrix (buffer mr), groups
  * GPS gs .. GPS gs + GPS - 1, in the stage layout above.  A 1-KB
  * instruction covers 64 / LPR rows, LPR lanes a row. */
 template <int BITS, int NR, bool WIDE, int GPS = 1>
-__device__ __forceinline__ void nmoe_stage_codes(uint32_t *stage, const uint32_t *mbase, int wpr, int row0, int gs,
-                                                 int j, int lane) {
+__device__ __forceinline__ void nmoe_stage_codes(uint32_t *stage, __amdgpu_buffer_rsrc_t mr, int wpr, int row0,
+                                                 int gs, int j, int lane) {
     using CR = nmoe_code_row<BITS, GPS>;
     constexpr uint32_t GW = nmoe_gwords<BITS>();
-    const uint32_t *gbase = mbase + (size_t)(GPS * gs) * NMOE_STRIPE * GW; /* the step's first group (uniform) */
+    const uint32_t soff = (uint32_t)(GPS * gs) * NMOE_STRIPE * GW * 4u; /* the step's first group (uniform) */
     if (WIDE) {
         const int row = (64 / CR::LPR) * j + lane / CR::LPR, part = (lane % CR::LPR) ^ CR::swz(row);
         const uint32_t u = (16u * part) / (4u * GW), w = ((16u * part) % (4u * GW)) / 4u; /* group of the step, word */
-        nmoe_dma<16>(gbase, 4u * (nmoe_stripe_word((uint32_t)(row0 + row), u, GW, (uint32_t)wpr) + w),
+        nmoe_dma<16>(mr, 4u * (nmoe_stripe_word((uint32_t)(row0 + row), u, GW, (uint32_t)wpr) + w), soff,
                      stage + 256 * j);
     } else {
         /* q2, one group: rows 16j + lane / 4, word lane % 4 */
         const int row = 16 * j + (lane >> 2);
-        nmoe_dma<4>(gbase, 4u * (nmoe_stripe_word((uint32_t)(row0 + row), 0u, GW, (uint32_t)wpr) + (lane & 3)),
+        nmoe_dma<4>(mr, 4u * (nmoe_stripe_word((uint32_t)(row0 + row), 0u, GW, (uint32_t)wpr) + (lane & 3)), soff,
                     stage + 64 * j);
     }
 }
@@ -1104,7 +1104,7 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
      * matrix cmat (gate for the first half of the wavefronts, up for the
      * second) */
     const int cmat = wave / (NW / 2);
-    const uint32_t *cbase = (const uint32_t *)(ex + (cmat == 0 ? L::gate_w : L::up_w)); /* stripe-major */
+    const __amdgpu_buffer_rsrc_t crs = nmoe_buffer((void *)(ex + (cmat == 0 ? L::gate_w : L::up_w))); /* stripe-major */
     const uint16_t *bias[2] = {(const uint16_t *)(ex + L::gate_b) + (size_t)nt * NT * G,
                                (const uint16_t *)(ex + L::up_b) + (size_t)nt * NT * G};
 
@@ -1142,18 +1142,18 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
 #pragma unroll
         for (int i = 0; i < AI; i++)
             row_off[i] = s_tok[8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3)] * (uint32_t)(NMOE_HIDDEN * 2);
-        const uint16_t *xpl[2] = {xhi, xlo};
+        const __amdgpu_buffer_rsrc_t xpl[2] = {nmoe_buffer((void *)xhi), nmoe_buffer((void *)xlo)};
         auto issue = [&](int gs, int st) {
 #pragma unroll
             for (int pl = 0; pl < XPL; pl++)
 #pragma unroll
                 for (int i = 0; i < AI; i++) {
                     const int j = wave + NW * i;
-                    nmoe_stage_rows(stage(st).a[pl], xpl[pl] + 64 * (GPS * gs + j / (MCH / 8)), row_off[i], j, lane);
+                    nmoe_stage_rows(stage(st).a[pl], xpl[pl], GPS * gs + j / (MCH / 8), row_off[i], j, lane);
                 }
 #pragma unroll
             for (int i = 0; i < CP::PER_WAVE; i++)
-                nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b + cmat * NT * CR::WPS, cbase, Q::WPR_G,
+                nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b + cmat * NT * CR::WPS, crs, Q::WPR_G,
                                                           nt * NT, gs, (CP::PER_WAVE * wave + i) % CPM, lane);
         };
         const int nb = (int)min((n - m0 + 15) / 16, (uint32_t)MB);
@@ -1456,7 +1456,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint8_t *ex = pack + (size_t)e * L::expert_size;
     const int rt0 = (NT / NW) * wave + col; /* tile row of column block nb: rt0 + 16 nb */
-    const uint32_t *cbase = (const uint32_t *)(ex + L::down_w); /* stripe-major */
+    const __amdgpu_buffer_rsrc_t crs = nmoe_buffer((void *)(ex + L::down_w)); /* stripe-major */
     const uint16_t *bias = (const uint16_t *)(ex + L::down_b) + (size_t)nt * NT * G;
 
     /* the tile in one form: up to MCH entries, GPS groups a ring step */
@@ -1492,7 +1492,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
         for (int i = 0; i < AI; i++)
             row_off[i] = (p0 + min(m0 + 8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3), n - 1)) *
                          (uint32_t)(NMOE_INTER * 2);
-        const uint16_t *apl[2] = {ahi, alo};
+        const __amdgpu_buffer_rsrc_t apl[2] = {nmoe_buffer((void *)ahi), nmoe_buffer((void *)alo)};
         /* a stage's act rows (2 AI loads) and its codes (CP::PER_WAVE loads) */
         auto issue_a = [&](int gs, int st) {
 #pragma unroll
@@ -1500,13 +1500,13 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
 #pragma unroll
                 for (int i = 0; i < AI; i++) {
                     const int j = wave + NW * i;
-                    nmoe_stage_rows(stage(st).a[pl], apl[pl] + 64 * (GPS * gs + j / (MCH / 8)), row_off[i], j, lane);
+                    nmoe_stage_rows(stage(st).a[pl], apl[pl], GPS * gs + j / (MCH / 8), row_off[i], j, lane);
                 }
         };
         auto issue_b = [&](int gs, int st) {
 #pragma unroll
             for (int i = 0; i < CP::PER_WAVE; i++)
-                nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b, cbase, Q::WPR_D, nt * NT, gs,
+                nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b, crs, Q::WPR_D, nt * NT, gs,
                                                           CP::PER_WAVE * wave + i, lane);
         };
         auto issue = [&](int gs, int st) {
