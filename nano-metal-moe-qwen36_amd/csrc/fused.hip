@@ -417,6 +417,15 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
     constexpr bool STK = XMODE == NMOE_XSTACK;
     constexpr bool NORM = XMODE == NMOE_XNORM || XMODE == NMOE_XBLOCK || STK; /* x = RMSNorm(h) in the block */
     constexpr bool BLK = XMODE == NMOE_XBLOCK;
+    /* x given: read once per block, whole lines a wavefront, into LDS in the
+     * workers' chunk order.  Loaded by each worker lane for itself (32 or 64
+     * consecutive columns, 64 to 256 bytes apart), every load touched a line
+     * a lane, eight wavefronts of them ahead of the block's router row in the
+     * CU's memory queue: a q2 step with fp32 x took 12.0 us, now 9.9; q4 with
+     * bf16 x 10.9, now 10.75.  The candidate wavefront still loads its own
+     * columns with its router row: from LDS they would wait for the barrier
+     * (q4 bf16 10.9, q2 fp32 10.05). */
+    constexpr bool XLDS = !NORM;
     __shared__ uint64_t s_tab[32];
     __shared__ float s_scratch[NMOE_EXPERTS];
     __shared__ float s_lg[NMOE_EXPERTS]; /* the token's logits, candidate -> exact wavefront */
@@ -432,7 +441,7 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
     __shared__ uint32_t s_epoch;
     __shared__ uint32_t s_ncand, s_confirm, s_lgok; /* control -> workers / control -> control hand-offs */
     __shared__ uint32_t s_bad; /* a wait of this block gave up: what it publishes is NaN */
-    __shared__ __align__(16) float s_h[NORM ? NMOE_HIDDEN : 4];
+    __shared__ __align__(16) float s_h[NMOE_HIDDEN];
     /* XBLOCK: the shared expert (gate values of this block's two rows, the
      * combining block's copy of all 512 activations, its 64 shared-down
      * rows and gate score) and the hand-offs between the wavefronts */
@@ -492,6 +501,9 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
             for (int i = 0; i < 8; i++) nwv[i] = nmoe_norm_weight(a.norm_w, 8 * tid + i, a.add_one);
         if (comb && tid < NMOE_FUSED_CHUNK) nxw = nmoe_norm_weight(a.next_w, crow, a.add_one);
     }
+    constexpr int XB = XMODE == NMOE_XBF16 ? 8 : 4; /* columns of a 16-byte load of x */
+    uint4 xw = make_uint4(0u, 0u, 0u, 0u);
+    if (XLDS && tid < NMOE_HIDDEN / XB) xw = ((const uint4 *)a.x)[tid];
     uint4 wv0[4]; /* the router row (not XSTACK: there it comes from LDS) */
     uint32_t wq0[4];
     uint16_t rsr0[4], rbr0[4];
@@ -644,6 +656,14 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
                 ((float4 *)s_h)[nmoe_act_slot<Q::CPL / 4>(c0) / 4] = v;
             }
         }
+    }
+    if (XLDS && tid < NMOE_HIDDEN / XB) {
+        float xf[8] = {__uint_as_float(xw.x), __uint_as_float(xw.y), __uint_as_float(xw.z), __uint_as_float(xw.w)};
+        if (XMODE == NMOE_XBF16) nmoe_unpack_bf16x8(xw, xf);
+#pragma unroll
+        for (int q = 0; q < XB / 4; q++)
+            ((float4 *)s_h)[nmoe_act_slot<Q::CPL / 4>(XB * tid + 4 * q) / 4] =
+                make_float4(xf[4 * q], xf[4 * q + 1], xf[4 * q + 2], xf[4 * q + 3]);
     }
     /* after the norm: thread 0 waits here for the launch epoch it loaded at
      * the start (a memory round trip), not before its loads of h */
@@ -1045,8 +1065,7 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
     /* the burst holds raw loads only: unpacking x or combining a scale with
      * its bias inside it would make the wave wait for those loads before
      * issuing the rest */
-    constexpr int XV = XMODE == NMOE_XBF16 ? Q::CPL / 8 : Q::CPL / 4; /* 16-byte x chunks per lane */
-    uint4 xr[XV];
+    constexpr int XV = Q::CPL / 4; /* 16-byte fp32 x chunks per lane */
     uint4 gwv[GSTEPS], uwv[GSTEPS], dwv[DSTEPS];
     uint32_t gsc[GSTEPS], gbi[GSTEPS], usc[GSTEPS], ubi[GSTEPS], dsc[DSTEPS], dbi[DSTEPS];
     /* the weights through a global-memory pointer (the stack form takes the
@@ -1104,11 +1123,6 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
     };
     uint32_t cand_g = 0;
     if (!ctrl && active) {
-        /* x first: loads retire in order, so G can start while down rows stream */
-        const uint4 *xp = (const uint4 *)a.x + gl * XV;
-        if (!NORM)
-#pragma unroll
-            for (int c = 0; c < XV; c++) xr[c] = xp[c];
         if (ROUTE) /* candidate g published by the control wavefront */
             nmoe_lds_wait_above(&s_cand[g], 0u, status, &s_bad, a.spin);
         const uint32_t cg = s_cand[g]; /* 0 only if that wait gave up */
@@ -1134,18 +1148,8 @@ __device__ __forceinline__ void nmoe_fused_body(nmoe_fused_args a, const nmoe_st
          * would wait for every load in flight: their direct LDS loads count
          * in the same counter) */
 #pragma unroll
-        for (int c = 0; c < XV; c++) {
-            if (NORM) {
-                *(float4 *)(xs + 4 * c) = ((const float4 *)s_h)[nmoe_act_slot<Q::CPL / 4>(4 * (gl * XV + c)) / 4];
-            } else if (XMODE == NMOE_XBF16) {
-                nmoe_unpack_bf16x8(xr[c], xs + 8 * c);
-            } else {
-                xs[4 * c] = __uint_as_float(xr[c].x);
-                xs[4 * c + 1] = __uint_as_float(xr[c].y);
-                xs[4 * c + 2] = __uint_as_float(xr[c].z);
-                xs[4 * c + 3] = __uint_as_float(xr[c].w);
-            }
-        }
+        for (int c = 0; c < XV; c++)
+            *(float4 *)(xs + 4 * c) = ((const float4 *)s_h)[nmoe_act_slot<Q::CPL / 4>(4 * (gl * XV + c)) / 4];
         gate_up();
         if (tid == 0) nmoe_tl_stamp(a.tl, ly, NMOE_TL_GU, actv[GSTEPS - 1]);
         if (NMOE_FUSED_DOWN_AFTER == 1) {
