@@ -1,5 +1,6 @@
-"""GPU: the many-token forms of the shared expert and the routers, through the
-C ABI, at the sizes where a tile, a grid or a dispatch rule ends."""
+"""GPU: the many-token forms of the shared expert and the routers and the
+grouped experts' work list, through the C ABI, at the sizes where a tile, a
+grid, a piece or a dispatch rule ends."""
 import numpy as np
 import pytest
 
@@ -134,3 +135,54 @@ def test_router_many_tokens_bit_exact(ctx, nh, kind, xdt, ntok, ne):
             B.oracle().orc_router_logits_q4(t[0].ctypes.data, t[1].ctypes.data, t[2].ctypes.data, xt.ctypes.data, ne,
                                             2048, o.ctypes.data)
         np.testing.assert_array_equal(got[tok].view(np.uint32), o.view(np.uint32))
+
+
+# entries an expert gets: either side of a 16-entry row block and of one, two
+# and three 64-entry pieces; one expert only; few experts of many pieces.  A
+# third of the tokens also have an entry on an expert of few entries; slots
+# left over hold indexes outside the layer
+@pytest.mark.parametrize("bits,xdt,counts,ntok", [
+    (4, "f32", [63, 64, 65, 127, 128, 129, 16, 17, 1, 2], 129), (2, "bf16", [64, 128, 192, 193, 15, 48, 49], 193),
+    (4, "bf16", [200], 200), (2, "f32", [1025, 1024, 961, 960, 449], 1025)])
+def test_grouped_pieces(nh, bits, xdt, counts, ntok):
+    """The grouped path (in one launch and in two: the same bits) against the
+    per-token kernels of the same call, relative L2 within 1e-4 as the
+    path's act planes (2^-17 a term) and fp32 sums allow, every token held
+    to 1e-3, and nothing written past the last token."""
+    rng = np.random.default_rng(len(counts) + ntok)
+    slots = np.full((ntok, 8), 0xFFFFFFFF, np.uint32)
+    fill = np.zeros(ntok, int)
+    for e, n in enumerate(counts):  # expert 11 e: n different tokens, the emptiest first
+        for t in np.argsort(fill + rng.random(ntok) * 0.5)[:n]:
+            slots[t, fill[t]] = 11 * e
+            fill[t] += 1
+    if len(counts) > 1:
+        for t in range(0, ntok, 3):
+            if fill[t] < 8:
+                slots[t, fill[t]] = 100 + t % 150
+    w = rng.dirichlet(np.ones(8), size=ntok).astype(np.float32)
+    c = nh.Context(0, max_tokens=ntok)
+    try:
+        c.synth_layer(1, bits, 5, 0.02 if bits == 4 else 0.05)
+        x, dx, dt = tokens(rng, c, nh, xdt, ntok)
+        h = rng.standard_normal((ntok, 2048)).astype(np.float32)
+        di, dw, dh = c.to_device(slots), c.to_device(w), c.to_device(h)
+        got = []
+        for gmin, one in ((8, True), (8, False), (1 << 20, True)):
+            c.set_grouped_min_tokens(gmin)
+            if not c.set_grouped_one_launch(one) and one and gmin == 8:
+                continue
+            out = c.to_device(np.full((ntok + 1, 2048), 7.5, np.float32))
+            c._check(c.experts(bits, 1, dx, dt, ntok, 8, di, dw, dh, out))
+            o = out.download(np.float32, (ntok + 1, 2048))
+            assert (o[ntok] == 7.5).all()
+            got.append(o[:ntok].astype(np.float64) - h)
+        assert c.device_status() == nh.OK
+    finally:
+        c.close()
+    want = got.pop()
+    for o in got:
+        np.testing.assert_array_equal(o, got[0])
+    rel = np.linalg.norm(got[0] - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-6)
+    print(f"[pieces] q{bits} {xdt} {ntok} tokens: worst token {rel.max():.2e}")
+    assert np.linalg.norm(got[0] - want) / np.linalg.norm(want) < 1e-4 and rel.max() < 1e-3
