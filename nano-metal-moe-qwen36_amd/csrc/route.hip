@@ -110,10 +110,11 @@ __global__ void __launch_bounds__(64) nmoe_router_q4_kernel(const uint32_t *__re
  * added, so it needs products of their own: v_mfma_f32_16x16x1_f32 (four
  * independent 16 x 16 products of one k each) gives b x and s x for four
  * columns at once.  bf16 x: s x is exact (16 significant bits) unless it is
- * subnormal, so fma(q, s x, b x) = fma(q s, x, b x) is a second MFMA on top
- * of b x, and only the add is left to the vector ALU.  fp32 x, and a bf16
- * chain that holds an x or s so small that s x may be subnormal: s x and b x
- * by MFMA, fma and add by the vector ALU.
+ * subnormal or overflows, so fma(q, s x, b x) = fma(q s, x, b x) is a second
+ * MFMA on top of b x, and only the add is left to the vector ALU.  fp32 x,
+ * and a bf16 chain that holds an x or s so small or so large that s x or q s
+ * may be subnormal or overflow: s x and b x by MFMA, fma and add by the
+ * vector ALU.
  *
  * Operands: lane l (row r = l % 16, kb = l / 16) loads columns 8 L .. 8 L + 7
  * of segment kb (512 columns a segment) of its row for chain L; a 4 x 4
@@ -208,12 +209,16 @@ __global__ void __launch_bounds__(512) nmoe_router_mm_kernel(const void *__restr
                 b[n][j] = nmoe_bf16f(bi[g]);
             }
     }
-    uint32_t smin = 0xffffffffu; /* q4, bf16 x: the wavefront's smallest nonzero |s| (as bits, less 1) */
+    /* q4, bf16 x: whether the lane holds an s outside 2^-63 .. 1 (0 apart) */
+    bool sout = false;
     if constexpr (Q4 && sizeof(XT) == 2) {
 #pragma unroll
         for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) smin = min(smin, (__float_as_uint(s[n][j]) & 0x7fffffffu) - 1u);
+            for (int j = 0; j < 4; j++) {
+                const uint32_t a = __float_as_uint(s[n][j]) & 0x7fffffffu;
+                sout = sout || a - 1u < ((127u - 63u) << 23) - 1u || a > (127u << 23);
+            }
     }
     /* the raw operands of two chains, loaded together (a row's 32 or 64
      * consecutive bytes) while the pair before them multiplies */
@@ -275,8 +280,10 @@ __global__ void __launch_bounds__(512) nmoe_router_mm_kernel(const void *__restr
                     wj[n][2] = q1[0];
                     wj[n][3] = q1[1];
                 }
-                /* s x exact for every s and x of the chain: no nonzero |x| below
-                 * 2^-70 or |s| below 2^-63 */
+                /* s x and q s exact for every s and x of the chain: no nonzero |x|
+                 * below 2^-70 and no nonzero |s| below 2^-63 (the lowest bit of
+                 * s x is then 2^-147 or more, the subnormals' 2^-149), no |s|
+                 * above 1 (no finite s x overflows) */
                 bool exact = false;
                 if constexpr (sizeof(XT) == 2) {
                     nmoe_rt_u16x2 xmin = {0xffff, 0xffff};
@@ -289,7 +296,7 @@ __global__ void __launch_bounds__(512) nmoe_router_mm_kernel(const void *__restr
                             xmin = __builtin_elementwise_min(xmin, __builtin_bit_cast(nmoe_rt_u16x2, u[i] & 0x7fff7fffu) - one);
                         }
                     }
-                    exact = __ballot(min(xmin.x, xmin.y) < ((127 - 70) << 7) - 1 || smin < ((127u - 63u) << 23) - 1u) == 0;
+                    exact = __ballot(min(xmin.x, xmin.y) < ((127 - 70) << 7) - 1 || sout) == 0;
                 }
                 if (c == 1) load(8 * wave + 2 * min(p + 1, 3));
                 const nmoe_rt_f32x16 z16 = {};

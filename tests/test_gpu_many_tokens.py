@@ -137,6 +137,51 @@ def test_router_many_tokens_bit_exact(ctx, nh, kind, xdt, ntok, ne):
         np.testing.assert_array_equal(got[tok].view(np.uint32), o.view(np.uint32))
 
 
+# the q4 terms' products at the ends of the exponent range, a 16 x 16 tile for
+# each: scales around 2 (s x overflows for the largest x), around 1e37 (q s
+# overflows) and below 2^-63 down to subnormals, with zero codes and scales and
+# biases of either sign; scales below 1 with the same x
+@pytest.mark.parametrize("xdt,ntok", [("bf16", 208), ("f32", 224)])
+def test_router_q4_extreme_products(ctx, nh, xdt, ntok):
+    """Bit for bit the few-token kernel's logits (NaN for NaN) and the oracle's."""
+    rng = np.random.default_rng(ntok)
+    w, s, b = q4_tensor(rng, 256, 2048, 2.0, 1)
+    w[::7] &= np.uint32(0x0F0F0F0F)  # half of the row's codes 0
+    f = B.bf16_to_f32(s).reshape(s.shape).copy()
+    for e, m in enumerate((1.0, 1e37, 1e-20, 1e-30, 1e-38)):
+        f[16 * e:16 * e + 16] = np.clip(f[16 * e:16 * e + 16], -8, 8) * np.float32(m)
+    f[80:96, ::5] = 0.0
+    f[96:128] = np.clip(f[96:128] * np.float32(0.2), -1, 1)
+    b = np.where(rng.random(s.shape) < 0.5, -8 * f.astype(np.float64), np.where(rng.random(s.shape) < 0.5, 0.0, f))
+    s, b = (B.f32_to_bf16(np.clip(v, -3e38, 3e38).astype(np.float32)).reshape(s.shape) for v in (f, b))
+    r = nh.Context.router_q4(*device_copy(ctx, (w, s, b), 1), 256)
+    x = rng.standard_normal((ntok, 2048)).astype(np.float32)
+    for t, m in enumerate((1e37, 8e37, 3e36, 1e20, 1.0, 1e-5, 1e-20, 1e-25, 1e-37, 1e-38)):
+        x[16 * t:16 * t + 16] = np.clip(x[16 * t:16 * t + 16], -4, 4) * np.float32(m)
+    x[0], x[1], x[2], x[16, ::3] = 3.3e38, 0.0, 0.0, 0.0
+    x[1, 77], x[2, 900] = 3e38, -1e38  # one term only: no other sign makes a NaN of an infinity
+    if xdt == "bf16":
+        xb = B.f32_to_bf16(x)
+        x, dx, dt, size = B.bf16_to_f32(xb).reshape(ntok, 2048), ctx.to_device(xb), nh.BF16, 2
+    else:
+        dx, dt, size = ctx.to_device(x), nh.F32, 4
+    assert np.isfinite(x).all() and np.isfinite(B.bf16_to_f32(s)).all() and np.isfinite(B.bf16_to_f32(b)).all()
+    lg, ref = ctx.alloc(ntok * 1024), ctx.alloc(ntok * 1024)
+    ctx._check(ctx.router_logits(r, dx, dt, ntok, lg))
+    for t0 in range(0, ntok, 64):
+        ctx._check(ctx.router_logits(r, dx.ptr + t0 * 2048 * size, dt, min(64, ntok - t0), ref.ptr + t0 * 1024))
+    got, want = lg.download(np.float32, (ntok, 256)), ref.download(np.float32, (ntok, 256))
+    assert np.isnan(want).any() and np.isinf(want).any() and np.isfinite(want).any()
+    for t in list(range(0, ntok, 16)) + [1, 2, ntok - 1]:
+        o, xt = np.zeros(256, np.float32), np.ascontiguousarray(x[t], np.float32)
+        B.oracle().orc_router_logits_q4(w.ctypes.data, s.ctypes.data, b.ctypes.data, xt.ctypes.data, 256, 2048,
+                                        o.ctypes.data)
+        np.testing.assert_array_equal(want[t], o)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    fine = ~np.isnan(want)
+    np.testing.assert_array_equal(got.view(np.uint32)[fine], want.view(np.uint32)[fine])
+
+
 # entries an expert gets: either side of a 16-entry row block and of one, two
 # and three 64-entry pieces; one expert only; few experts of many pieces.  A
 # third of the tokens also have an entry on an expert of few entries; slots
