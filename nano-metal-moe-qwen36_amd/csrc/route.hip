@@ -386,29 +386,50 @@ static void nmoe_router_mm_launch(const nmoe_hip_router *router, const void *x, 
                        router->scales, router->biases, (const XT *)x, ntok, ne, logits);
 }
 
-/* Tokens from which the matrix form runs.  One 16 x 16 tile takes a CU about
- * 4 us (bf16 router) or 12 to 16 us (q4), whatever the token count, so the
- * one-row-a-wavefront kernels, which spread few tokens over the whole chip,
- * stay ahead up to there: bf16 router 6.8 against 8.2 us (fp32 x) and 4.9
- * against 6.4 us (bf16 x) at 64 tokens, 20.1 against 8.6 and 12.9 against
- * 6.9 us at 251; q4 router 7.5 against 17.5 and 6.6 against 12.6 us at 64,
- * 22.1 against 17.9 and 17.9 against 12.9 us at 251. */
-#define NMOE_ROUTER_MM_MIN 96
-#define NMOE_ROUTER_MM_MIN_Q4 192
+/* Whether the matrix form runs.  It takes the time of its rounds of 16 x 16
+ * tiles over the 256 CUs, whatever they hold; the one-row-a-wavefront kernels
+ * that of ntok (ne + c) terms, c for the loads of x.  256 experts, us, one row
+ * a wavefront against the matrix form, either side of each line:
+ *   bf16 router, fp32 x   8.3 / 8.1 at 88 tokens, 8.9 / 8.1 at 96
+ *   bf16 router, bf16 x   5.9 / 6.2 at 96, 6.3 / 6.25 at 104; second round
+ *                         12.6 / 10.4 at 257
+ *   q4 router, fp32 x     17.4 / 17.6 at 200, 18.1 / 17.6 at 208; second
+ *                         round 28.4 / 29.7 at 352, 30.7 / 29.7 at 384; third
+ *                         42.0 / 41.5 at 513
+ *   q4 router, bf16 x     12.5 / 13.0 at 192, 13.6 / 13.1 at 200; second
+ *                         21.8 / 22.2 at 352, 22.7 / 22.3 at 368; third 30.0 /
+ *                         30.4 at 513, 34.8 / 30.8 at 600
+ * and fewer experts, from which c: 64 experts, fp32 x, 7.8 / 8.2 at 300 tokens
+ * (bf16 router), 13.1 / 17.4 at 512 and 24.3 / 17.6 at 1,000 (q4); 16 experts,
+ * 5.0 / 8.2 at 512 and 12.2 / 8.3 at 1,000, 12.6 / 17.4 at 1,000 and 23.0 /
+ * 17.6 at 2,048; 2 experts, bf16 router, 4.0 / 7.4 at 2,048. */
+static bool nmoe_router_mm_pays(bool q4, bool bf, int ntok, int ne) {
+    if (ne < 4) return false;
+    const int c = q4 ? (bf ? 11 : 20) : (bf ? 8 : 18);
+    const long tokens = (long)ntok * (ne + c) / (NMOE_EXPERTS + c); /* of 256 experts */
+    if (!q4) return tokens >= (bf ? 104 : 96);
+    const long tiles = (long)((ne + 15) / 16) * ((ntok + 15) / 16);
+    return tokens >= (tiles <= 256 ? (bf ? 200 : 208) : (bf ? 368 : 384));
+}
 
 template <typename XT>
 static void nmoe_router_mm(const nmoe_hip_router *router, const void *x, int ntok, float *logits, hipStream_t s) {
-    /* the tile whose grid over 256 experts is about one round of the 256 CUs:
-     * a larger tile reads each row of w and x less often, a smaller one
-     * leaves no CU idle.  bf16 router, fp32 x, 16x16 / 32x32 / 32x64 tiles
-     * (us): 8.6 / 15 / 25 at 251 tokens, 34 / 23 / 28 at 1,000, 125 / 80 / 61
-     * at 4,096.  The q4 router is bound by its vector instructions and keeps
-     * the smallest (the larger ones spill). */
+    /* the smallest tile whose grid is one round of the 256 CUs (or, with
+     * rows of x few enough, two): a larger tile reads each row of w and x less
+     * often, a smaller one leaves no CU idle.  bf16 router, fp32 x, 256
+     * experts, 16x16 / 32x32 / 32x64 tiles (us): 8.6 / 15 / 25 at 251 tokens,
+     * 17.2 / 17.6 at 512, 20.8 / 17.7 at 513, 34 / 23 / 28 at 1,000, 125 / 80
+     * / 61 at 4,096; bf16 x 12.0 / 14.0 at 272, 13.0 / 14.1 at 512; 128
+     * experts 20.5 / 17.9 at 1,000; 64 experts, 32x32 / 32x64, 18.7 / 25.2 at
+     * 2,048 and 31.3 / 27.3 at 4,096.  The q4 router is bound by its vector
+     * instructions and keeps the smallest (the larger ones spill). */
+    const int ne = router->num_experts;
+    auto tiles = [&](int rows, int cols) { return (long)((ntok + rows - 1) / rows) * ((ne + cols - 1) / cols); };
     if (router->kind == NMOE_HIP_ROUTER_Q4)
         nmoe_router_mm_launch<true, XT, 1, 1>(router, x, ntok, logits, s);
-    else if (ntok <= 256)
+    else if (ntok <= 512 || tiles(16, 16) <= 256)
         nmoe_router_mm_launch<false, XT, 1, 1>(router, x, ntok, logits, s);
-    else if (ntok <= 1024)
+    else if (ntok <= 2048 && tiles(32, 32) <= 256)
         nmoe_router_mm_launch<false, XT, 2, 2>(router, x, ntok, logits, s);
     else
         nmoe_router_mm_launch<false, XT, 2, 4>(router, x, ntok, logits, s);
@@ -471,7 +492,7 @@ int nmoe_check_x(nmoe_hip_ctx *ctx, const void *x, int x_dtype, int ntok) {
 /* The router launch with its arguments already checked. */
 extern "C" hipError_t nmoe_router_logits_launch(const nmoe_hip_router *router, const void *x, int x_dtype, int ntok,
                                                float *logits, hipStream_t s) {
-    if (ntok >= (router->kind == NMOE_HIP_ROUTER_Q4 ? NMOE_ROUTER_MM_MIN_Q4 : NMOE_ROUTER_MM_MIN)) {
+    if (nmoe_router_mm_pays(router->kind == NMOE_HIP_ROUTER_Q4, x_dtype == NMOE_HIP_BF16, ntok, router->num_experts)) {
         if (x_dtype == NMOE_HIP_BF16)
             nmoe_router_mm<uint16_t>(router, x, ntok, logits, s);
         else

@@ -91,12 +91,16 @@ def test_shared_expert_many_tokens(ctx, nh, xdt, ntok):
     assert rel(got[pick], want_so) < 2e-6 and rel(got_g[pick], want_gr) < 2e-6
 
 
-# one row a wavefront up to 95 (q4: 191) tokens, then tiles of 16 x 16, 32 x 32
-# (from 257) and 32 x 64 (from 1,025), with ragged last tiles of tokens and experts
+# one row a wavefront for few terms, then tiles of 16 x 16, 32 x 32 (from 513
+# tokens) and 32 x 64 (from 1,025), with ragged last tiles of tokens and experts:
+# either side of each line of the rule, for few experts too
 @pytest.mark.parametrize("kind,xdt,ntok,ne", [
     ("bf16", "f32", 96, 256), ("bf16", "bf16", 241, 250), ("bf16", "f32", 257, 256), ("bf16", "bf16", 290, 33),
     ("bf16", "bf16", 1025, 256), ("bf16", "f32", 1041, 241), ("q4", "f32", 192, 256), ("q4", "bf16", 193, 256),
-    ("q4", "f32", 300, 17), ("q4", "bf16", 1025, 250)])
+    ("q4", "f32", 300, 17), ("q4", "bf16", 1025, 250), ("bf16", "bf16", 104, 256), ("bf16", "bf16", 512, 256),
+    ("bf16", "f32", 513, 256), ("bf16", "bf16", 1100, 33), ("bf16", "f32", 1100, 120), ("q4", "f32", 208, 256),
+    ("q4", "f32", 257, 256), ("q4", "f32", 384, 256), ("q4", "bf16", 200, 256), ("q4", "bf16", 384, 250),
+    ("q4", "f32", 1000, 40), ("q4", "bf16", 1100, 40)])
 def test_router_many_tokens_bit_exact(ctx, nh, kind, xdt, ntok, ne):
     """The matrix form's logits bit for bit the few-token kernel's (the same
     tokens 64 at a time) and, for a few tokens, the oracle's; subnormal, huge,
