@@ -121,9 +121,12 @@ __device__ __forceinline__ int nmoe_act_swz(int col) {
  * activations' loads go out ahead of the weights', and staging and summing
  * them runs while the weights arrive.  With a branch a slot, each slot's
  * index was waited for before the next one's load, and the activations came
- * one load at a time (4 tokens, q4: 9.4 us, now 7.6).
+ * one load at a time (4 tokens, q4, 8 experts: 9.4 us, now 7.6).
+ * KU: the slots a block is laid out for, 2 for k <= 2.  Laid out for 8, one
+ * expert a token pays for the others' loads and stores (7 tokens, q4, k = 1:
+ * 5.8 us, with a branch a slot 4.4; both launches 10.5 and 9.7, now 8.5).
  * out[t][r] = h_mid[t][r] + sum_s w[t][s] * y_s[r] (+ sigmoid(g_t) * shared[t][r]). */
-template <int BITS>
+template <int BITS, int KU>
 __global__ void __launch_bounds__(256) nmoe_down_combine_kernel(
     const uint8_t *__restrict__ pack, int k, const uint32_t *__restrict__ idx, const float *__restrict__ wts,
     const float *__restrict__ act, const float *h_mid, const float *__restrict__ shared_out,
@@ -132,31 +135,31 @@ __global__ void __launch_bounds__(256) nmoe_down_combine_kernel(
     using L = nmoe_layout<BITS>;
     constexpr int RPW = NMOE_WAVE / Q::LPR_D;            /* rows per wavefront: 4 (q4) / 8 (q2) */
     constexpr int RPB = RPW * NMOE_DC_WAVES;
-    __shared__ float4 act_s[NMOE_MAX_K * NMOE_INTER / 4];
-    __shared__ float asum_s[NMOE_MAX_K][Q::LPR_D];
+    __shared__ float4 act_s[KU * NMOE_INTER / 4];
+    __shared__ float asum_s[KU][Q::LPR_D];
     const int t = blockIdx.y;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int sub = lane / Q::LPR_D, l = lane % Q::LPR_D;
     const int row = blockIdx.x * RPB + wave * RPW + sub;
 
-    constexpr int AQ = NMOE_MAX_K * (NMOE_INTER / 4) / 256;
+    constexpr int AQ = KU * (NMOE_INTER / 4) / 256;
     const float4 *a4 = (const float4 *)(act + (size_t)t * NMOE_MAX_K * NMOE_INTER);
     float4 av[AQ];
 #pragma unroll
     for (int q = 0; q < AQ; q++) av[q] = a4[min((int)threadIdx.x + 256 * q, k * (NMOE_INTER / 4) - 1)];
-    uint4 dw[NMOE_MAX_K];
-    uint32_t ds[NMOE_MAX_K], db[NMOE_MAX_K];
-    float wk[NMOE_MAX_K];
+    uint4 dw[KU];
+    uint32_t ds[KU], db[KU];
+    float wk[KU];
     const int grp = l * Q::CPL / NMOE_GROUP;
-    uint32_t ei[NMOE_MAX_K];
+    uint32_t ei[KU];
 #pragma unroll
-    for (int s = 0; s < NMOE_MAX_K; s++) {
+    for (int s = 0; s < KU; s++) {
         const size_t i = (size_t)t * NMOE_MAX_K + min(s, k - 1);
         ei[s] = idx[i];
         wk[s] = wts[i];
     }
 #pragma unroll
-    for (int s = 0; s < NMOE_MAX_K; s++) {
+    for (int s = 0; s < KU; s++) {
         /* an index outside the layer is an invalid slot: weight 0, as for
          * a failed expert read in the reference (runtime.m:2977-2981) */
         wk[s] = ei[s] < NMOE_EXPERTS ? wk[s] : 0.0f;
@@ -173,7 +176,7 @@ __global__ void __launch_bounds__(256) nmoe_down_combine_kernel(
         act_s[s * (NMOE_INTER / 4) + (nmoe_act_swz<BITS>(col) >> 2)] = av[q];
     }
     __syncthreads();
-    static_assert(NMOE_MAX_K * Q::LPR_D <= 256, "one sum a thread");
+    static_assert(KU * Q::LPR_D <= 256 && KU * (NMOE_INTER / 4) % 256 == 0, "one sum a thread, whole loads");
     if ((int)threadIdx.x < k * Q::LPR_D) {
         const int s = threadIdx.x / Q::LPR_D, ll = threadIdx.x % Q::LPR_D;
         float a = 0.0f;
@@ -188,7 +191,7 @@ __global__ void __launch_bounds__(256) nmoe_down_combine_kernel(
 
     float moe = 0.0f;
 #pragma unroll
-    for (int s = 0; s < NMOE_MAX_K; s++) {
+    for (int s = 0; s < KU; s++) {
         if (s < k) {
             float xs[Q::CPL];
 #pragma unroll
@@ -272,8 +275,12 @@ static hipError_t nmoe_launch_experts_act(const uint8_t *pack, const void *x, in
     if (e != hipSuccess) return e;
     constexpr int RPB = (NMOE_WAVE / Q::LPR_D) * NMOE_DC_WAVES;
     dim3 g2(NMOE_HIDDEN / RPB, ntok);
-    hipLaunchKernelGGL((nmoe_down_combine_kernel<BITS>), g2, dim3(256), 0, s, pack, k, idx, w, act, h_mid, shared_out,
-                       shared_gate_raw, out);
+    if (k <= 2)
+        hipLaunchKernelGGL((nmoe_down_combine_kernel<BITS, 2>), g2, dim3(256), 0, s, pack, k, idx, w, act, h_mid,
+                           shared_out, shared_gate_raw, out);
+    else
+        hipLaunchKernelGGL((nmoe_down_combine_kernel<BITS, NMOE_MAX_K>), g2, dim3(256), 0, s, pack, k, idx, w, act,
+                           h_mid, shared_out, shared_gate_raw, out);
     return hipGetLastError();
 }
 

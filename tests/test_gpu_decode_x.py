@@ -51,7 +51,8 @@ def test_given_x_types_agree(bits, k):
         np.testing.assert_array_equal(o.view(np.uint32), outs[0].view(np.uint32))
 
 
-@pytest.mark.parametrize("bits,k,ntok", [(4, 1, 2), (4, 6, 7), (4, 7, 3), (2, 1, 7), (2, 6, 3), (2, 8, 7)])
+@pytest.mark.parametrize("bits,k,ntok", [(4, 1, 2), (4, 6, 7), (4, 7, 3), (2, 1, 7), (2, 6, 3), (2, 8, 7),
+                                         (4, 2, 7), (4, 3, 5), (2, 2, 5), (2, 3, 2)])
 def test_few_tokens_unused_slots(bits, k, ntok):
     """The per-token kernels: slots past k hold indexes outside the layer and
     NaN weights, one used slot an index outside the layer (weight 0); x, idx
