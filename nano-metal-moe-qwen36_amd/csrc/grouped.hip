@@ -84,11 +84,14 @@ __host__ __device__ constexpr int nmoe_work_places(int n) {
 #ifndef NMOE_GROUPED_NW
 #define NMOE_GROUPED_NW 4
 #endif
-/* The small form: an expert of at most NMOE_SMALL_PASS entries (batched
- * decode leaves most experts with a few) runs one pass of one 16-row block
- * whose ring steps take NMOE_SMALL_GPS groups at a time, so each weight row
- * is read 64 B a step instead of 32 B and the A stage holds 16 rows, not
- * 64.  Built with four-wavefront blocks (one A load per wavefront a step). */
+/* The small form: a piece of at most NMOE_SMALL_PASS entries (batched
+ * decode leaves most experts with a few) runs as one 16-row block whose ring
+ * steps take NMOE_SMALL_GPS groups at a time, so each weight row is read 64 B
+ * a step instead of 32 B and the A stage holds 16 rows, not 64.  Both GEMMs
+ * have it, in one launch and in two (without it in the two-launch down
+ * kernel: 3 to 8 % of a call of up to 256 tokens, 94.4 and 88.7 us at 48
+ * tokens, bf16 x, q4; up to 2 % of 4,096 skewed q2 tokens).  Built with
+ * four-wavefront blocks (one A load per wavefront a step). */
 #define NMOE_SMALL_PASS 16
 #define NMOE_SMALL_GPS 2
 __host__ __device__ constexpr bool nmoe_small_form(int nw) { return nw == 4; }
@@ -1663,7 +1666,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     }
     };
     /* block-uniform: the piece's entry count picks the form */
-    if constexpr (nmoe_small_form(NW) && WAIT) {
+    if constexpr (nmoe_small_form(NW)) {
         if (n <= (uint32_t)NMOE_SMALL_PASS) {
             run(std::integral_constant<int, NMOE_SMALL_PASS>{}, std::integral_constant<int, NMOE_SMALL_GPS>{});
             return;
