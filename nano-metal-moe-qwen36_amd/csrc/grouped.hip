@@ -1111,8 +1111,11 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
     const int e = (int)min(rk.x, (uint32_t)(NMOE_EXPERTS - 1));
     const uint32_t p0 = min(rk.y, (uint32_t)nrows);
     uint32_t n = min(min(rk.z, (uint32_t)NMOE_MCHUNK), (uint32_t)nrows - p0);
+    /* (two launches, bf16 x) n as a value of no known bound: with the bound of
+     * 64 the q2 tile spills 53 registers (the call 24 % slower); fp32 x runs
+     * 1 % faster with it */
+    if constexpr (!COUNT && XPL == 1) n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
     if (n == 0u) return;
-    asm("" : "+s"(n));
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kb = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint8_t *ex = pack + (size_t)e * L::expert_size;
@@ -1125,7 +1128,7 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
     const uint16_t *bias[2] = {(const uint16_t *)(ex + L::gate_b) + (size_t)nt * NT * G,
                                (const uint16_t *)(ex + L::up_b) + (size_t)nt * NT * G};
 
-    /* the tile in one form: up to MCH entries, GPS groups a ring step */
+    /* the tile in one form: n <= MCH entries, GPS groups a ring step */
     auto run = [&](auto mch_c, auto gps_c) {
     constexpr int MCH = decltype(mch_c)::value, GPS = decltype(gps_c)::value;
     constexpr int MB = MCH / 16;                /* row blocks of a whole piece */
@@ -1149,207 +1152,205 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
 #pragma unroll
         for (int b2 = 0; b2 < NB; b2++) coff[u][b2] = nmoe_code_off<BITS, GPS>(rt0 + 16 * b2, u, kb);
 
-    for (uint32_t m0 = 0; m0 < n; m0 += MCH) { /* once */
-        if (tid < MCH) s_tok[tid] = min(perm[p0 + min(m0 + tid, n - 1)], (uint32_t)nrows - 1u) / (uint32_t)k;
+    if (tid < MCH) s_tok[tid] = min(perm[p0 + min((uint32_t)tid, n - 1)], (uint32_t)nrows - 1u) / (uint32_t)k;
+    nmoe_lds_barrier();
+    /* this lane's A row for instruction j = wave + NW i (rows 8j .. 8j+7
+     * of the stage plane: group j / (MCH / 8), entries 8 (j % (MCH / 8))
+     * + lane / 8) */
+    uint32_t row_off[AI];
+#pragma unroll
+    for (int i = 0; i < AI; i++)
+        row_off[i] = s_tok[8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3)] * (uint32_t)(NMOE_HIDDEN * 2);
+    const __amdgpu_buffer_rsrc_t xpl[2] = {nmoe_buffer((void *)xhi), nmoe_buffer((void *)xlo)};
+    auto issue = [&](int gs, int st) {
+#pragma unroll
+        for (int pl = 0; pl < XPL; pl++)
+#pragma unroll
+            for (int i = 0; i < AI; i++) {
+                const int j = wave + NW * i;
+                nmoe_stage_rows(stage(st).a[pl], xpl[pl], GPS * gs + j / (MCH / 8), row_off[i], j, lane);
+            }
+#pragma unroll
+        for (int i = 0; i < CP::PER_WAVE; i++)
+            nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b + cmat * NT * CR::WPS, crs, Q::WPR_G,
+                                                      nt * NT, gs, (CP::PER_WAVE * wave + i) % CPM, lane);
+    };
+    const int nb = (int)min((n + 15) / 16, (uint32_t)MB);
+    nmoe_f32x4 acc[2][NB][MB];
+    {
+        /* The correction's operands go out first and the first ring
+         * stages right after them: loads retire in order, so the
+         * small loads then return without waiting for the stages,
+         * and the correction's MFMAs run while the stages stream in.
+         * A lane = (entry col, groups 8kb .. 8kb+7), B lane = (row
+         * col, the same groups): a lane's eight groups are contiguous
+         * (one 16-byte load per part of xs, one of the biases, one
+         * LDS read of the scales). */
+        constexpr int PER = 2 * NT * G / 8 / NTH;
+        static_assert(PER * NTH == 2 * NT * G / 8, "scale chunks split evenly over the threads");
+        /* the tile's scales straight into LDS: wavefront w's q-th 1 KB
+         * at uint4 NTH q + 64w */
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            /* LDS chunk i = (mat, chunk, row) <- global chunk row * G/8 + chunk of the matrix */
+            const int i = tid + NTH * q, mat = i / (NT * G / 8), j = i % (NT * G / 8);
+            const int ch = j / NT, row = j % NT;
+            const uint4 *src = (const uint4 *)(ex + (mat == 0 ? L::gate_s : L::up_s) + (size_t)nt * NT * G * 2) +
+                               row * (G / 8) + ch;
+            __builtin_amdgcn_global_load_lds(
+                (const void *)src, (nmoe_lds_void *)((uint4 *)&s_s[0][0][0][0] + NTH * q + 64 * wave), 16, 0, 0);
+        }
+        uint4 xq[MB][3];
+        uint4 bv[2][NB];
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+                xq[mb][p] = *(const uint4 *)(xs3 + ((size_t)s_tok[16 * mb + col] * 3 + p) * G + 8 * kb);
+#pragma unroll
+        for (int mat = 0; mat < 2; mat++)
+#pragma unroll
+            for (int b2 = 0; b2 < NB; b2++)
+                bv[mat][b2] = *(const uint4 *)(bias[mat] + (rt0 + 16 * b2) * G + 8 * kb);
+#pragma unroll
+        for (int st = 0; st < NS - 1; st++) issue(st, st);
+        /* scales, xs and biases have landed once only the stages'
+         * loads are in flight; then every wavefront's scales are in
+         * LDS */
+        nmoe_wait_vm<(NS - 1) * (XPL * AI + CP::PER_WAVE)>();
         nmoe_lds_barrier();
-        /* this lane's A row for instruction j = wave + NW i (rows 8j .. 8j+7
-         * of the stage plane: group j / (MCH / 8), entries 8 (j % (MCH / 8))
-         * + lane / 8) */
-        uint32_t row_off[AI];
 #pragma unroll
-        for (int i = 0; i < AI; i++)
-            row_off[i] = s_tok[8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3)] * (uint32_t)(NMOE_HIDDEN * 2);
-        const __amdgpu_buffer_rsrc_t xpl[2] = {nmoe_buffer((void *)xhi), nmoe_buffer((void *)xlo)};
-        auto issue = [&](int gs, int st) {
+        for (int mat = 0; mat < 2; mat++)
 #pragma unroll
-            for (int pl = 0; pl < XPL; pl++)
+            for (int b2 = 0; b2 < NB; b2++) {
+                const uint4 sv = *(const uint4 *)&s_s[mat][kb][rt0 + 16 * b2][0];
 #pragma unroll
-                for (int i = 0; i < AI; i++) {
-                    const int j = wave + NW * i;
-                    nmoe_stage_rows(stage(st).a[pl], xpl[pl], GPS * gs + j / (MCH / 8), row_off[i], j, lane);
+                for (int mb = 0; mb < MB; mb++) {
+                    nmoe_f32x4 a = nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    if (mb < nb) {
+                        nmoe_f32x4 t = nmoe_mfma16(xq[mb][0], sv, nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                        t = nmoe_mfma16(xq[mb][1], sv, t);
+                        t = nmoe_mfma16(xq[mb][2], sv, t);
+                        a = nmoe_mfma16(xq[mb][0], bv[mat][b2], a);
+                        a = nmoe_mfma16(xq[mb][1], bv[mat][b2], a);
+                        a = nmoe_mfma16(xq[mb][2], bv[mat][b2], a);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) a[i] = __builtin_fmaf(-128.0f, t[i], a[i]);
+                    }
+                    acc[mat][b2][mb] = a;
+                }
+            }
+    }
+    auto step = [&](int gs, const int st, const bool ahead) {
+        nmoe_ring_step_barrier<XPL * AI + CP::PER_WAVE, G / GPS, NS>(gs);
+        if (ahead) issue(gs + NS - 1, (st + NS - 1) % NS);
+        /* the step's scales: one bf16, or both groups' in one word */
+        uint32_t sw[2][NB];
+#pragma unroll
+        for (int mat = 0; mat < 2; mat++)
+#pragma unroll
+            for (int b2 = 0; b2 < NB; b2++) {
+                const uint16_t *sp = &s_s[mat][(GPS * gs) >> 3][rt0 + 16 * b2][(GPS * gs) & 7];
+                sw[mat][b2] = GPS == 2 ? *(const uint32_t *)sp : (uint32_t)*sp;
+            }
+#pragma unroll
+        for (int u = 0; u < GPS; u++) {
+            uint4 bq[2][NB][2];
+            float sg[2][NB];
+#pragma unroll
+            for (int mat = 0; mat < 2; mat++)
+#pragma unroll
+                for (int b2 = 0; b2 < NB; b2++) {
+                    uint32_t w0, w1;
+                    /* kept apart: two reads merged into one instruction lose
+                     * the stage they belong to, and then wait for every stage */
+                    if (u + mat + b2 > 0) asm volatile("" ::: "memory");
+                    nmoe_code_read<BITS>(stage(st).b + mat * NT * CR::WPS, coff[u][b2], w0, w1);
+                    nmoe_codes_bf16<BITS>(w0, w1, bq[mat][b2][0], bq[mat][b2][1]);
+                    sg[mat][b2] = nmoe_bf16f((uint16_t)(sw[mat][b2] >> (16 * u)));
                 }
 #pragma unroll
-            for (int i = 0; i < CP::PER_WAVE; i++)
-                nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b + cmat * NT * CR::WPS, crs, Q::WPR_G,
-                                                          nt * NT, gs, (CP::PER_WAVE * wave + i) % CPM, lane);
-        };
-        const int nb = (int)min((n - m0 + 15) / 16, (uint32_t)MB);
-        nmoe_f32x4 acc[2][NB][MB];
-        {
-            /* The correction's operands go out first and the first ring
-             * stages right after them: loads retire in order, so the
-             * small loads then return without waiting for the stages,
-             * and the correction's MFMAs run while the stages stream in.
-             * A lane = (entry col, groups 8kb .. 8kb+7), B lane = (row
-             * col, the same groups): a lane's eight groups are contiguous
-             * (one 16-byte load per part of xs, one of the biases, one
-             * LDS read of the scales). */
-            constexpr int PER = 2 * NT * G / 8 / NTH;
-            static_assert(PER * NTH == 2 * NT * G / 8, "scale chunks split evenly over the threads");
-            /* the tile's scales straight into LDS: wavefront w's q-th 1 KB
-             * at uint4 NTH q + 64w */
+            for (int mb = 0; mb < MB; mb++) {
+                if (mb < nb) {
+                    uint4 a[XPL][2];
 #pragma unroll
-            for (int q = 0; q < PER; q++) {
-                /* LDS chunk i = (mat, chunk, row) <- global chunk row * G/8 + chunk of the matrix */
-                const int i = tid + NTH * q, mat = i / (NT * G / 8), j = i % (NT * G / 8);
-                const int ch = j / NT, row = j % NT;
-                const uint4 *src = (const uint4 *)(ex + (mat == 0 ? L::gate_s : L::up_s) + (size_t)nt * NT * G * 2) +
-                                   row * (G / 8) + ch;
-                __builtin_amdgcn_global_load_lds(
-                    (const void *)src, (nmoe_lds_void *)((uint4 *)&s_s[0][0][0][0] + NTH * q + 64 * wave), 16, 0, 0);
+                    for (int pl = 0; pl < XPL; pl++)
+                        nmoe_stage_operand(stage(st).a[pl], MCH * u + 16 * mb + col, kb, a[pl][0], a[pl][1]);
+#pragma unroll
+                    for (int mat = 0; mat < 2; mat++)
+#pragma unroll
+                        for (int b2 = 0; b2 < NB; b2++) {
+                            nmoe_f32x4 pp =
+                                nmoe_mfma16(a[0][0], bq[mat][b2][0], nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                            pp = nmoe_mfma16(a[0][1], bq[mat][b2][1], pp);
+                            if (XPL == 2) {
+                                pp = nmoe_mfma16(a[XPL - 1][0], bq[mat][b2][0], pp);
+                                pp = nmoe_mfma16(a[XPL - 1][1], bq[mat][b2][1], pp);
+                            }
+#pragma unroll
+                            for (int i = 0; i < 4; i++)
+                                acc[mat][b2][mb][i] = __builtin_fmaf(sg[mat][b2], pp[i], acc[mat][b2][mb][i]);
+                        }
+                }
             }
-            uint4 xq[MB][3];
-            uint4 bv[2][NB];
+        }
+    };
+    nmoe_ring_run<G / GPS, NS>(step);
+    {
+        /* epilogue: act = SiLU(gate) * up as hi + lo bf16, in the down
+         * kernel's operand order; group sums of act rows (a down group
+         * is 64 act columns, WPD wavefronts of this tile) */
+        float part_sum[MB][4] = {};
+        /* the act planes as buffers: a scalar base and a 32-bit lane
+         * offset per store (no 64-bit address arithmetic) */
+        const __amdgpu_buffer_rsrc_t rhi = nmoe_buffer(ahi), rlo = nmoe_buffer(alo);
+        /* byte offset of this lane's act column in a row, per column block */
+        uint32_t cb[NB];
+#pragma unroll
+        for (int b2 = 0; b2 < NB; b2++) {
+            const int r = nt * NT + rt0 + 16 * b2; /* act column */
+            cb[b2] = 2u * (uint32_t)(16 * (r >> 4) + nmoe_kperm_inv<BITS>(r & 15));
+        }
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            if (mb >= nb) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t m = 16 * mb + 4 * kb + i;
+                /* the row's byte offset from the (uniform) plane base */
+                const uint32_t ro = (p0 + min(m, n - 1)) * (uint32_t)(NMOE_INTER * 2);
+                float part = 0.0f;
+#pragma unroll
+                for (int b2 = 0; b2 < NB; b2++) {
+                    const float av = nmoe_silu_fast(acc[0][b2][mb][i]) * acc[1][b2][mb][i];
+                    const uint32_t h = nmoe_bf16_cvt(av);
+                    const uint32_t l = nmoe_bf16_cvt(av - nmoe_bf16f(h));
+                    part = part + (nmoe_bf16f(h) + nmoe_bf16f(l));
+                    if (m < n) {
+                        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)h, rhi, ro + cb[b2], 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)l, rlo, ro + cb[b2], 0, 0);
+                    }
+                }
+                /* the wavefront's 2 NB x 16 act columns of this row */
+                part_sum[mb][i] = nmoe_dpp_group_sum<16>(part);
+            }
+        }
+        if (col == 0)
 #pragma unroll
             for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-                for (int p = 0; p < 3; p++)
-                    xq[mb][p] = *(const uint4 *)(xs3 + ((size_t)s_tok[16 * mb + col] * 3 + p) * G + 8 * kb);
+                for (int i = 0; i < 4; i++) s_as[wave][16 * mb + 4 * kb + i] = part_sum[mb][i];
+    }
+    nmoe_lds_barrier();
+    constexpr int DG = NT / 64;  /* down groups per tile */
+    constexpr int WPD = NW / DG; /* wavefronts per down group */
+    if (tid < DG * MCH) {
+        const int dg = tid / MCH, row = tid % MCH;
+        const uint32_t m = row;
+        float t = s_as[WPD * dg][row];
 #pragma unroll
-            for (int mat = 0; mat < 2; mat++)
-#pragma unroll
-                for (int b2 = 0; b2 < NB; b2++)
-                    bv[mat][b2] = *(const uint4 *)(bias[mat] + (rt0 + 16 * b2) * G + 8 * kb);
-#pragma unroll
-            for (int st = 0; st < NS - 1; st++) issue(st, st);
-            /* scales, xs and biases have landed once only the stages'
-             * loads are in flight; then every wavefront's scales are in
-             * LDS */
-            nmoe_wait_vm<(NS - 1) * (XPL * AI + CP::PER_WAVE)>();
-            nmoe_lds_barrier();
-#pragma unroll
-            for (int mat = 0; mat < 2; mat++)
-#pragma unroll
-                for (int b2 = 0; b2 < NB; b2++) {
-                    const uint4 sv = *(const uint4 *)&s_s[mat][kb][rt0 + 16 * b2][0];
-#pragma unroll
-                    for (int mb = 0; mb < MB; mb++) {
-                        nmoe_f32x4 a = nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                        if (mb < nb) {
-                            nmoe_f32x4 t = nmoe_mfma16(xq[mb][0], sv, nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-                            t = nmoe_mfma16(xq[mb][1], sv, t);
-                            t = nmoe_mfma16(xq[mb][2], sv, t);
-                            a = nmoe_mfma16(xq[mb][0], bv[mat][b2], a);
-                            a = nmoe_mfma16(xq[mb][1], bv[mat][b2], a);
-                            a = nmoe_mfma16(xq[mb][2], bv[mat][b2], a);
-#pragma unroll
-                            for (int i = 0; i < 4; i++) a[i] = __builtin_fmaf(-128.0f, t[i], a[i]);
-                        }
-                        acc[mat][b2][mb] = a;
-                    }
-                }
-        }
-        auto step = [&](int gs, const int st, const bool ahead) {
-            nmoe_ring_step_barrier<XPL * AI + CP::PER_WAVE, G / GPS, NS>(gs);
-            if (ahead) issue(gs + NS - 1, (st + NS - 1) % NS);
-            /* the step's scales: one bf16, or both groups' in one word */
-            uint32_t sw[2][NB];
-#pragma unroll
-            for (int mat = 0; mat < 2; mat++)
-#pragma unroll
-                for (int b2 = 0; b2 < NB; b2++) {
-                    const uint16_t *sp = &s_s[mat][(GPS * gs) >> 3][rt0 + 16 * b2][(GPS * gs) & 7];
-                    sw[mat][b2] = GPS == 2 ? *(const uint32_t *)sp : (uint32_t)*sp;
-                }
-#pragma unroll
-            for (int u = 0; u < GPS; u++) {
-                uint4 bq[2][NB][2];
-                float sg[2][NB];
-#pragma unroll
-                for (int mat = 0; mat < 2; mat++)
-#pragma unroll
-                    for (int b2 = 0; b2 < NB; b2++) {
-                        uint32_t w0, w1;
-                        /* kept apart: two reads merged into one instruction lose
-                         * the stage they belong to, and then wait for every stage */
-                        if (u + mat + b2 > 0) asm volatile("" ::: "memory");
-                        nmoe_code_read<BITS>(stage(st).b + mat * NT * CR::WPS, coff[u][b2], w0, w1);
-                        nmoe_codes_bf16<BITS>(w0, w1, bq[mat][b2][0], bq[mat][b2][1]);
-                        sg[mat][b2] = nmoe_bf16f((uint16_t)(sw[mat][b2] >> (16 * u)));
-                    }
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++) {
-                    if (mb < nb) {
-                        uint4 a[XPL][2];
-#pragma unroll
-                        for (int pl = 0; pl < XPL; pl++)
-                            nmoe_stage_operand(stage(st).a[pl], MCH * u + 16 * mb + col, kb, a[pl][0], a[pl][1]);
-#pragma unroll
-                        for (int mat = 0; mat < 2; mat++)
-#pragma unroll
-                            for (int b2 = 0; b2 < NB; b2++) {
-                                nmoe_f32x4 pp =
-                                    nmoe_mfma16(a[0][0], bq[mat][b2][0], nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-                                pp = nmoe_mfma16(a[0][1], bq[mat][b2][1], pp);
-                                if (XPL == 2) {
-                                    pp = nmoe_mfma16(a[XPL - 1][0], bq[mat][b2][0], pp);
-                                    pp = nmoe_mfma16(a[XPL - 1][1], bq[mat][b2][1], pp);
-                                }
-#pragma unroll
-                                for (int i = 0; i < 4; i++)
-                                    acc[mat][b2][mb][i] = __builtin_fmaf(sg[mat][b2], pp[i], acc[mat][b2][mb][i]);
-                            }
-                    }
-                }
-            }
-        };
-        nmoe_ring_run<G / GPS, NS>(step);
-        {
-            /* epilogue: act = SiLU(gate) * up as hi + lo bf16, in the down
-             * kernel's operand order; group sums of act rows (a down group
-             * is 64 act columns, WPD wavefronts of this tile) */
-            float part_sum[MB][4] = {};
-            /* the act planes as buffers: a scalar base and a 32-bit lane
-             * offset per store (no 64-bit address arithmetic) */
-            const __amdgpu_buffer_rsrc_t rhi = nmoe_buffer(ahi), rlo = nmoe_buffer(alo);
-            /* byte offset of this lane's act column in a row, per column block */
-            uint32_t cb[NB];
-#pragma unroll
-            for (int b2 = 0; b2 < NB; b2++) {
-                const int r = nt * NT + rt0 + 16 * b2; /* act column */
-                cb[b2] = 2u * (uint32_t)(16 * (r >> 4) + nmoe_kperm_inv<BITS>(r & 15));
-            }
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                if (mb >= nb) continue;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t m = m0 + 16 * mb + 4 * kb + i;
-                    /* the row's byte offset from the (uniform) plane base */
-                    const uint32_t ro = (p0 + min(m, n - 1)) * (uint32_t)(NMOE_INTER * 2);
-                    float part = 0.0f;
-#pragma unroll
-                    for (int b2 = 0; b2 < NB; b2++) {
-                        const float av = nmoe_silu_fast(acc[0][b2][mb][i]) * acc[1][b2][mb][i];
-                        const uint32_t h = nmoe_bf16_cvt(av);
-                        const uint32_t l = nmoe_bf16_cvt(av - nmoe_bf16f(h));
-                        part = part + (nmoe_bf16f(h) + nmoe_bf16f(l));
-                        if (m < n) {
-                            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)h, rhi, ro + cb[b2], 0, 0);
-                            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)l, rlo, ro + cb[b2], 0, 0);
-                        }
-                    }
-                    /* the wavefront's 2 NB x 16 act columns of this row */
-                    part_sum[mb][i] = nmoe_dpp_group_sum<16>(part);
-                }
-            }
-            if (col == 0)
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) s_as[wave][16 * mb + 4 * kb + i] = part_sum[mb][i];
-        }
-        nmoe_lds_barrier();
-        constexpr int DG = NT / 64;  /* down groups per tile */
-        constexpr int WPD = NW / DG; /* wavefronts per down group */
-        if (tid < DG * MCH) {
-            const int dg = tid / MCH, row = tid % MCH;
-            const uint32_t m = m0 + row;
-            float t = s_as[WPD * dg][row];
-#pragma unroll
-            for (int q = 1; q < WPD; q++) t = t + s_as[WPD * dg + q][row];
-            if (m < n) as[(size_t)(p0 + m) * (NMOE_INTER / NMOE_GROUP) + DG * nt + dg] = t;
-        }
+        for (int q = 1; q < WPD; q++) t = t + s_as[WPD * dg + q][row];
+        if (m < n) as[(size_t)(p0 + m) * (NMOE_INTER / NMOE_GROUP) + DG * nt + dg] = t;
     }
     };
     /* block-uniform: the piece's entry count picks the form */
@@ -1466,8 +1467,10 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     const int e = (int)min(rk.x, (uint32_t)(NMOE_EXPERTS - 1));
     const uint32_t p0 = min(rk.y, (uint32_t)nrows);
     uint32_t n = min(min(rk.z, (uint32_t)NMOE_MCHUNK), (uint32_t)nrows - p0);
+    /* (two launches) as in the gate/up tile: a call of 1,000 to 4,096 tokens 2
+     * to 3 % slower with the bound known */
+    if constexpr (!WAIT) n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
     if (n == 0u) return;
-    asm("" : "+s"(n));
     static_assert(!WAIT || NS == 3, "the split prologue's waits are written for three stages");
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kb = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1476,7 +1479,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     const __amdgpu_buffer_rsrc_t crs = nmoe_buffer((void *)(ex + L::down_w)); /* stripe-major */
     const uint16_t *bias = (const uint16_t *)(ex + L::down_b) + (size_t)nt * NT * G;
 
-    /* the tile in one form: up to MCH entries, GPS groups a ring step */
+    /* the tile in one form: n <= MCH entries, GPS groups a ring step */
     auto run = [&](auto mch_c, auto gps_c) {
     constexpr int MCH = decltype(mch_c)::value, GPS = decltype(gps_c)::value;
     constexpr int MB = MCH / 16;           /* row blocks of a whole piece */
@@ -1496,171 +1499,169 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     for (int u = 0; u < GPS; u++)
 #pragma unroll
         for (int b2 = 0; b2 < NB; b2++) coff[u][b2] = nmoe_code_off<BITS, GPS>(rt0 + 16 * b2, u, kb);
-    for (uint32_t m0 = 0; m0 < n; m0 += MCH) { /* once */
-        /* the chunk's output slots, stored to LDS after the stages are issued
-         * (so that this load's wait does not hold them back) and visible
-         * after the barrier below */
-        const uint32_t qv = tid < MCH ? min(perm[p0 + min(m0 + tid, n - 1)], (uint32_t)nrows - 1u) : 0u;
-        /* this lane's A row for instruction j = wave + NW i (group
-         * j / (MCH / 8) of the step): act row p0 + 8 (j % (MCH / 8)) +
-         * lane / 8 */
-        uint32_t row_off[AI];
+    /* the chunk's output slots, stored to LDS after the stages are issued
+     * (so that this load's wait does not hold them back) and visible
+     * after the barrier below */
+    const uint32_t qv = tid < MCH ? min(perm[p0 + min((uint32_t)tid, n - 1)], (uint32_t)nrows - 1u) : 0u;
+    /* this lane's A row for instruction j = wave + NW i (group
+     * j / (MCH / 8) of the step): act row p0 + 8 (j % (MCH / 8)) +
+     * lane / 8 */
+    uint32_t row_off[AI];
 #pragma unroll
-        for (int i = 0; i < AI; i++)
-            row_off[i] = (p0 + min(m0 + 8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3), n - 1)) *
-                         (uint32_t)(NMOE_INTER * 2);
-        const __amdgpu_buffer_rsrc_t apl[2] = {nmoe_buffer((void *)ahi), nmoe_buffer((void *)alo)};
-        /* a stage's act rows (2 AI loads) and its codes (CP::PER_WAVE loads) */
-        auto issue_a = [&](int gs, int st) {
+    for (int i = 0; i < AI; i++)
+        row_off[i] = (p0 + min((uint32_t)(8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3)), n - 1)) *
+                     (uint32_t)(NMOE_INTER * 2);
+    const __amdgpu_buffer_rsrc_t apl[2] = {nmoe_buffer((void *)ahi), nmoe_buffer((void *)alo)};
+    /* a stage's act rows (2 AI loads) and its codes (CP::PER_WAVE loads) */
+    auto issue_a = [&](int gs, int st) {
 #pragma unroll
-            for (int pl = 0; pl < 2; pl++)
+        for (int pl = 0; pl < 2; pl++)
 #pragma unroll
-                for (int i = 0; i < AI; i++) {
-                    const int j = wave + NW * i;
-                    nmoe_stage_rows(stage(st).a[pl], apl[pl], GPS * gs + j / (MCH / 8), row_off[i], j, lane);
-                }
-        };
-        auto issue_b = [&](int gs, int st) {
-#pragma unroll
-            for (int i = 0; i < CP::PER_WAVE; i++)
-                nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b, crs, Q::WPR_D, nt * NT, gs,
-                                                          CP::PER_WAVE * wave + i, lane);
-        };
-        auto issue = [&](int gs, int st) {
-            issue_a(gs, st);
-            issue_b(gs, st);
-        };
-        const int nb = (int)min((n - m0 + 15) / 16, (uint32_t)MB);
-        nmoe_f32x4 acc[NB][MB];
-        {
-            /* as in the gate/up kernel: the correction's operands
-             * (scales straight into LDS, one 16-byte chunk a thread), then the first ring stages, then a wait that
-             * leaves only the stages in flight.
-             * A lane = (entry col, groups 2kb + tq), B lane = (row col,
-             * groups 2kb + tq) */
-            static_assert(NT * G / 8 % 64 == 0 && NT * G / 8 <= 64 * NW, "at most one scale chunk per thread");
-            if (NT * G / 8 == 64 * NW || tid < NT * G / 8) /* wavefront-uniform */
-                __builtin_amdgcn_global_load_lds(
-                    (const void *)((const uint4 *)(ex + L::down_s + (size_t)nt * NT * G * 2) + tid),
-                    (nmoe_lds_void *)((uint4 *)&s_s[0][0] + 64 * wave), 16, 0, 0);
-            float2 av[MB];
-            uint32_t bv[NB];
-            auto load_av = [&]() {
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++) {
-                    const float *ap = as + (size_t)(p0 + min(m0 + 16 * mb + col, n - 1)) * G + 2 * kb;
-                    if constexpr (WAIT)
-                        av[mb] = __builtin_bit_cast(float2, __hip_atomic_load((nmoe_g64 *)ap, __ATOMIC_RELAXED,
-                                                                              __HIP_MEMORY_SCOPE_AGENT));
-                    else
-                        av[mb] = *(const float2 *)ap;
-                }
-            };
-            if constexpr (WAIT) {
-                /* the weights first (they do not wait for the gate/up
-                 * tiles): biases and the first stages' codes; then the wait
-                 * for the piece's gate/up tiles (a
-                 * barrier that leaves the loads in flight); then the act
-                 * side: group sums and the first stages' act rows.  The wait
-                 * below leaves only stage 1's act rows in flight, so stage 0
-                 * is complete before the ring's first step. */
-#pragma unroll
-                for (int b2 = 0; b2 < NB; b2++) bv[b2] = *(const uint32_t *)(bias + (rt0 + 16 * b2) * G + 2 * kb);
-#pragma unroll
-                for (int st = 0; st < NS - 1; st++) issue_b(st, st);
-                if (tid == 0) {
-                    /* the fourth word: the piece's place in the gate/up order */
-                    nmoe_wait_tiles(done + min(rk.w, (uint32_t)ne - 1u), (uint32_t)gu_tiles, sync, spin);
-                    nmoe_gtl_stamp(tl, NMOE_GTL_READY);
-                }
-                nmoe_lds_barrier();
-                load_av();
-#pragma unroll
-                for (int st = 0; st < NS - 1; st++) issue_a(st, st);
-                nmoe_wait_vm<(NS - 2) * 2 * AI>();
-            } else {
-                load_av();
-#pragma unroll
-                for (int b2 = 0; b2 < NB; b2++) bv[b2] = *(const uint32_t *)(bias + (rt0 + 16 * b2) * G + 2 * kb);
-#pragma unroll
-                for (int st = 0; st < NS - 1; st++) issue(st, st);
-                nmoe_wait_vm<(NS - 1) * (2 * AI + CP::PER_WAVE)>();
+            for (int i = 0; i < AI; i++) {
+                const int j = wave + NW * i;
+                nmoe_stage_rows(stage(st).a[pl], apl[pl], GPS * gs + j / (MCH / 8), row_off[i], j, lane);
             }
-            if (tid < MCH) s_q[tid] = qv;
-            nmoe_lds_barrier(); /* the scales and s_q */
-            float cv[NB][G / 4];
+    };
+    auto issue_b = [&](int gs, int st) {
 #pragma unroll
-            for (int b2 = 0; b2 < NB; b2++) {
-                const uint32_t sw = *(const uint32_t *)&s_s[rt0 + 16 * b2][2 * kb];
-                cv[b2][0] = __uint_as_float(bv[b2] << 16) - 128.0f * __uint_as_float(sw << 16);
-                cv[b2][1] = __uint_as_float(bv[b2] & 0xffff0000u) - 128.0f * __uint_as_float(sw & 0xffff0000u);
+        for (int i = 0; i < CP::PER_WAVE; i++)
+            nmoe_stage_codes<BITS, NT, CP::WIDE, GPS>(stage(st).b, crs, Q::WPR_D, nt * NT, gs,
+                                                      CP::PER_WAVE * wave + i, lane);
+    };
+    auto issue = [&](int gs, int st) {
+        issue_a(gs, st);
+        issue_b(gs, st);
+    };
+    const int nb = (int)min((n + 15) / 16, (uint32_t)MB);
+    nmoe_f32x4 acc[NB][MB];
+    {
+        /* as in the gate/up kernel: the correction's operands
+         * (scales straight into LDS, one 16-byte chunk a thread), then the first ring stages, then a wait that
+         * leaves only the stages in flight.
+         * A lane = (entry col, groups 2kb + tq), B lane = (row col,
+         * groups 2kb + tq) */
+        static_assert(NT * G / 8 % 64 == 0 && NT * G / 8 <= 64 * NW, "at most one scale chunk per thread");
+        if (NT * G / 8 == 64 * NW || tid < NT * G / 8) /* wavefront-uniform */
+            __builtin_amdgcn_global_load_lds(
+                (const void *)((const uint4 *)(ex + L::down_s + (size_t)nt * NT * G * 2) + tid),
+                (nmoe_lds_void *)((uint4 *)&s_s[0][0] + 64 * wave), 16, 0, 0);
+        float2 av[MB];
+        uint32_t bv[NB];
+        auto load_av = [&]() {
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++) acc[b2][mb] = nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int mb = 0; mb < MB; mb++) {
+                const float *ap = as + (size_t)(p0 + min((uint32_t)(16 * mb + col), n - 1)) * G + 2 * kb;
+                if constexpr (WAIT)
+                    av[mb] = __builtin_bit_cast(float2, __hip_atomic_load((nmoe_g64 *)ap, __ATOMIC_RELAXED,
+                                                                          __HIP_MEMORY_SCOPE_AGENT));
+                else
+                    av[mb] = *(const float2 *)ap;
             }
+        };
+        if constexpr (WAIT) {
+            /* the weights first (they do not wait for the gate/up
+             * tiles): biases and the first stages' codes; then the wait
+             * for the piece's gate/up tiles (a
+             * barrier that leaves the loads in flight); then the act
+             * side: group sums and the first stages' act rows.  The wait
+             * below leaves only stage 1's act rows in flight, so stage 0
+             * is complete before the ring's first step. */
 #pragma unroll
-            for (int tq = 0; tq < G / 4; tq++)
+            for (int b2 = 0; b2 < NB; b2++) bv[b2] = *(const uint32_t *)(bias + (rt0 + 16 * b2) * G + 2 * kb);
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++)
-                    if (mb < nb)
+            for (int st = 0; st < NS - 1; st++) issue_b(st, st);
+            if (tid == 0) {
+                /* the fourth word: the piece's place in the gate/up order */
+                nmoe_wait_tiles(done + min(rk.w, (uint32_t)ne - 1u), (uint32_t)gu_tiles, sync, spin);
+                nmoe_gtl_stamp(tl, NMOE_GTL_READY);
+            }
+            nmoe_lds_barrier();
+            load_av();
 #pragma unroll
-                        for (int b2 = 0; b2 < NB; b2++)
-                            acc[b2][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(tq == 0 ? av[mb].x : av[mb].y,
-                                                                               cv[b2][tq], acc[b2][mb], 0, 0, 0);
+            for (int st = 0; st < NS - 1; st++) issue_a(st, st);
+            nmoe_wait_vm<(NS - 2) * 2 * AI>();
+        } else {
+            load_av();
+#pragma unroll
+            for (int b2 = 0; b2 < NB; b2++) bv[b2] = *(const uint32_t *)(bias + (rt0 + 16 * b2) * G + 2 * kb);
+#pragma unroll
+            for (int st = 0; st < NS - 1; st++) issue(st, st);
+            nmoe_wait_vm<(NS - 1) * (2 * AI + CP::PER_WAVE)>();
         }
-        auto step = [&](int gs, const int st, const bool ahead) {
-            nmoe_ring_step_barrier<2 * AI + CP::PER_WAVE, G / GPS, NS>(gs);
-            if (ahead) issue(gs + NS - 1, (st + NS - 1) % NS);
-            /* the step's scales: one bf16, or both groups' in one word */
-            uint32_t sw[NB];
+        if (tid < MCH) s_q[tid] = qv;
+        nmoe_lds_barrier(); /* the scales and s_q */
+        float cv[NB][G / 4];
+#pragma unroll
+        for (int b2 = 0; b2 < NB; b2++) {
+            const uint32_t sw = *(const uint32_t *)&s_s[rt0 + 16 * b2][2 * kb];
+            cv[b2][0] = __uint_as_float(bv[b2] << 16) - 128.0f * __uint_as_float(sw << 16);
+            cv[b2][1] = __uint_as_float(bv[b2] & 0xffff0000u) - 128.0f * __uint_as_float(sw & 0xffff0000u);
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) acc[b2][mb] = nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int tq = 0; tq < G / 4; tq++)
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+                if (mb < nb)
+#pragma unroll
+                    for (int b2 = 0; b2 < NB; b2++)
+                        acc[b2][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(tq == 0 ? av[mb].x : av[mb].y,
+                                                                           cv[b2][tq], acc[b2][mb], 0, 0, 0);
+    }
+    auto step = [&](int gs, const int st, const bool ahead) {
+        nmoe_ring_step_barrier<2 * AI + CP::PER_WAVE, G / GPS, NS>(gs);
+        if (ahead) issue(gs + NS - 1, (st + NS - 1) % NS);
+        /* the step's scales: one bf16, or both groups' in one word */
+        uint32_t sw[NB];
+#pragma unroll
+        for (int b2 = 0; b2 < NB; b2++) {
+            const uint16_t *sp = &s_s[rt0 + 16 * b2][GPS * gs];
+            sw[b2] = GPS == 2 ? *(const uint32_t *)sp : (uint32_t)*sp;
+        }
+#pragma unroll
+        for (int u = 0; u < GPS; u++) {
+            uint4 bq[NB][2];
+            float sg[NB];
 #pragma unroll
             for (int b2 = 0; b2 < NB; b2++) {
-                const uint16_t *sp = &s_s[rt0 + 16 * b2][GPS * gs];
-                sw[b2] = GPS == 2 ? *(const uint32_t *)sp : (uint32_t)*sp;
+                uint32_t w0, w1;
+                /* kept apart, as in the gate/up kernel */
+                if (u + b2 > 0) asm volatile("" ::: "memory");
+                nmoe_code_read<BITS>(stage(st).b, coff[u][b2], w0, w1);
+                nmoe_codes_bf16<BITS>(w0, w1, bq[b2][0], bq[b2][1]);
+                sg[b2] = nmoe_bf16f((uint16_t)(sw[b2] >> (16 * u)));
             }
 #pragma unroll
-            for (int u = 0; u < GPS; u++) {
-                uint4 bq[NB][2];
-                float sg[NB];
+            for (int mb = 0; mb < MB; mb++) {
+                if (mb < nb) {
+                    uint4 h0, h1, l0, l1;
+                    nmoe_stage_operand(stage(st).a[0], MCH * u + 16 * mb + col, kb, h0, h1);
+                    nmoe_stage_operand(stage(st).a[1], MCH * u + 16 * mb + col, kb, l0, l1);
 #pragma unroll
-                for (int b2 = 0; b2 < NB; b2++) {
-                    uint32_t w0, w1;
-                    /* kept apart, as in the gate/up kernel */
-                    if (u + b2 > 0) asm volatile("" ::: "memory");
-                    nmoe_code_read<BITS>(stage(st).b, coff[u][b2], w0, w1);
-                    nmoe_codes_bf16<BITS>(w0, w1, bq[b2][0], bq[b2][1]);
-                    sg[b2] = nmoe_bf16f((uint16_t)(sw[b2] >> (16 * u)));
-                }
+                    for (int b2 = 0; b2 < NB; b2++) {
+                        nmoe_f32x4 pp = nmoe_mfma16(h0, bq[b2][0], nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                        pp = nmoe_mfma16(h1, bq[b2][1], pp);
+                        pp = nmoe_mfma16(l0, bq[b2][0], pp);
+                        pp = nmoe_mfma16(l1, bq[b2][1], pp);
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++) {
-                    if (mb < nb) {
-                        uint4 h0, h1, l0, l1;
-                        nmoe_stage_operand(stage(st).a[0], MCH * u + 16 * mb + col, kb, h0, h1);
-                        nmoe_stage_operand(stage(st).a[1], MCH * u + 16 * mb + col, kb, l0, l1);
-#pragma unroll
-                        for (int b2 = 0; b2 < NB; b2++) {
-                            nmoe_f32x4 pp = nmoe_mfma16(h0, bq[b2][0], nmoe_f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-                            pp = nmoe_mfma16(h1, bq[b2][1], pp);
-                            pp = nmoe_mfma16(l0, bq[b2][0], pp);
-                            pp = nmoe_mfma16(l1, bq[b2][1], pp);
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                acc[b2][mb][i] = __builtin_fmaf(sg[b2], pp[i], acc[b2][mb][i]);
-                        }
+                        for (int i = 0; i < 4; i++)
+                            acc[b2][mb][i] = __builtin_fmaf(sg[b2], pp[i], acc[b2][mb][i]);
                     }
                 }
             }
-        };
-        nmoe_ring_run<G / GPS, NS>(step);
+        }
+    };
+    nmoe_ring_run<G / GPS, NS>(step);
 #pragma unroll
-        for (int b2 = 0; b2 < NB; b2++) {
-            const int r = nt * NT + rt0 + 16 * b2;
+    for (int b2 = 0; b2 < NB; b2++) {
+        const int r = nt * NT + rt0 + 16 * b2;
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
+        for (int mb = 0; mb < MB; mb++) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t m = m0 + 16 * mb + 4 * kb + i;
-                    if (mb < nb && m < n) y[(size_t)s_q[m - m0] * NMOE_HIDDEN + r] = acc[b2][mb][i];
-                }
+            for (int i = 0; i < 4; i++) {
+                const uint32_t m = 16 * mb + 4 * kb + i;
+                if (mb < nb && m < n) y[(size_t)s_q[m] * NMOE_HIDDEN + r] = acc[b2][mb][i];
             }
         }
     }
