@@ -302,9 +302,9 @@ __device__ __forceinline__ void nmoe_dispatch_entries(const nmoe_entry_src &s, i
 /* The scatter's LDS counts: per chunk of the first NMOE_DISPATCH_PRE and
  * wavefront, the entries of each expert (then their first places), and
  * the short pieces' size classes.  Cleared by nmoe_dispatch_count. */
-struct __align__(16) nmoe_scatter_lds {
+struct nmoe_scatter_lds {
     uint32_t wc[NMOE_DISPATCH_PRE][4][NMOE_EXPERTS + 1];
-    __align__(16) uint32_t wbk[4][8]; /* each wavefront's short pieces of each size class */
+    uint32_t wbk[4][8]; /* each wavefront's short pieces of each size class */
 };
 
 /* D1: h = expert histogram of entry slice b of nd (in LDS). */
@@ -368,7 +368,7 @@ __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src,
                                                       uint32_t r1, nmoe_scatter_lds &sl) {
     __shared__ uint32_t s_base[NMOE_EXPERTS];
     __shared__ uint32_t s_scan[4]; /* the wavefronts' totals */
-    __shared__ __align__(16) uint32_t s_full[4]; /* and their whole pieces */
+    __shared__ uint32_t s_full[4]; /* and their whole pieces */
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = ntok * src.k;
     const int per = (n + nd - 1) / nd, q0 = b * per, q1 = min(n, (b + 1) * per);
     /* thread e: total of expert e and its count in the slices before b,
@@ -484,24 +484,15 @@ __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src,
         }
     }
     if (b == 0) {
-        /* pieces of each class, those of the earlier wavefronts, and the
-         * expert's first whole piece (16-byte LDS reads) */
-        uint32_t cnt[4] = {}, prev = 0u, fpos = finc - full, nfull = 0u;
-        const uint4 fv = *(const uint4 *)s_full;
-        const uint32_t fw[4] = {fv.x, fv.y, fv.z, fv.w};
+        uint32_t cnt[4], fpos = finc - full, nfull = 0u; /* pieces of each class; the expert's first whole piece */
 #pragma unroll
         for (int w = 0; w < 4; w++) {
-            const uint4 v = *(const uint4 *)sl.wbk[w];
-            const uint32_t c[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                cnt[i] += c[i];
-                prev += w < wave && i == bk ? c[i] : 0u;
-            }
-            fpos += w < wave ? fw[w] : 0u;
-            nfull += fw[w];
+            fpos += w < wave ? s_full[w] : 0u;
+            nfull += s_full[w];
         }
-        const uint32_t nbig = nfull + cnt[0] + cnt[1] + cnt[2], rounds = (uint32_t)ne >> 3;
+#pragma unroll
+        for (int i = 0; i < 4; i++) cnt[i] = sl.wbk[0][i] + sl.wbk[1][i] + sl.wbk[2][i] + sl.wbk[3][i];
+        const uint32_t nbig = nfull + cnt[0] + cnt[1] + cnt[2], nwork = nbig + cnt[3], rounds = (uint32_t)ne >> 3;
         /* the place of position pos (its fourth word: the place itself), and
          * the same piece in the down tiles' order after it */
         auto put = [&](uint32_t pos, uint32_t first, uint32_t entries) {
@@ -514,11 +505,14 @@ __device__ __forceinline__ void nmoe_dispatch_scatter(const nmoe_entry_src &src,
         };
         for (uint32_t j = 0; j < min(full, (uint32_t)ne); j++) put(fpos + j, off + NMOE_MCHUNK * j, NMOE_MCHUNK);
         if (rem != 0u) {
-            uint32_t pos = nfull + prev + brk;
+            uint32_t pos = nfull + brk;
 #pragma unroll
             for (int i = 0; i < 3; i++) pos += i < bk ? cnt[i] : 0u;
+#pragma unroll
+            for (int w = 0; w < 3; w++) pos += w < wave ? sl.wbk[w][bk] : 0u;
             put(pos, off + NMOE_MCHUNK * full, rem);
         }
+        for (uint32_t pos = nwork + (uint32_t)tid; pos < (uint32_t)ne; pos += 256u) put(pos, 0u, 0u);
     }
     /* slices of more than NMOE_DISPATCH_PRE chunks: the others one at a
      * time, counted in sl.wc[0] */
@@ -671,10 +665,6 @@ __global__ void __launch_bounds__(256) nmoe_grouped_prep_kernel(const uint32_t *
      * path) from a count no tiles can reach */
     if (done != NULL && b == 0)
         for (int i = threadIdx.x; i < ne; i += 256) done[i] = i == skew ? 0x8000u : 0u;
-    /* every place of both lists empty; the pieces are put after the block's
-     * barriers (here the stores are done while the routing is waited for) */
-    if (b == 0)
-        for (int i = threadIdx.x; i < 2 * ne; i += 256) rank[i] = make_uint4(0u, 0u, 0u, 0u);
     const int nr = ROUTED ? (ntok + 3) / 4 : 0; /* routing blocks */
     if (ROUTED && b >= nd && b < nd + nr) {
         __shared__ float s_sm[4][NMOE_EXPERTS];
