@@ -448,6 +448,10 @@ __global__ void __launch_bounds__(256, 2) nmoe_shared_mm_kernel(nmoe_sh_ws ws, i
                 }
             }
             if (GU) {
+                /* (the product of as[] fused into the first add of its sum would
+                 * round differently in the two lanes of a pair, and a token's
+                 * sums then depend on whether it sits in an even or an odd row) */
+#pragma clang fp contract(off)
                 /* act column 32 n + 16 q + col of tokens 4 kb .. + 3: slice n,
                  * k 16 q + col of the down product's operand */
                 const int k = 16 * q + col;

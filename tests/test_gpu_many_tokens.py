@@ -91,6 +91,26 @@ def test_shared_expert_many_tokens(ctx, nh, xdt, ntok):
     assert rel(got[pick], want_so) < 2e-6 and rel(got_g[pick], want_gr) < 2e-6
 
 
+@pytest.mark.parametrize("xdt,ntok", [("f32", 67), ("bf16", 300)])
+def test_shared_expert_place_in_the_call(ctx, nh, xdt, ntok):
+    """A token's matrix-form output does not depend on its place in the call:
+    the tokens from the first, second, fourth and eighteenth on, bit for bit."""
+    rng = np.random.default_rng(ntok)
+    t = [q4_tensor(rng, r, k, s, 1) for r, k, s in
+         ((512, 2048, 0.004), (512, 2048, 0.004), (2048, 512, 0.008), (1, 2048, 0.004))]
+    desc = nh.Context.shared_expert_desc(*(device_copy(ctx, q, 1) for q in t))
+    _, dx, dt = tokens(rng, ctx, nh, xdt, ntok)
+    got = []
+    for first in (0, 1, 3, 17):
+        n = ntok - first
+        so, gr = ctx.alloc(n * 8192), ctx.alloc(n * 4)
+        ctx._check(ctx.shared_expert(desc, dx.ptr + first * 2048 * (4 if dt == nh.F32 else 2), dt, n, so, gr))
+        got.append((so.download(np.uint32, (n, 2048))[17 - first:], gr.download(np.uint32, n)[17 - first:]))
+    for so, gr in got[1:]:
+        np.testing.assert_array_equal(so, got[0][0])
+        np.testing.assert_array_equal(gr, got[0][1])
+
+
 # one row a wavefront for few terms, then tiles of 16 x 16, 32 x 32 (from 513
 # tokens) and 32 x 64 (from 1,025), with ragged last tiles of tokens and experts:
 # either side of each line of the rule, for few experts too
