@@ -75,8 +75,10 @@ typedef struct nmoe_hip_ctx nmoe_hip_ctx;
 /* ---- context (replaces nmoe_backend_create/destroy, backend.h:55-56, and the
  *      one-time buffer set-up NMOEInitExpertIOBuffers, runtime.m:1542-1584) */
 
-/* max_tokens bounds ntok for every later call; scratch for that many tokens
- * is allocated here, once. */
+/* max_tokens (1..65536) bounds ntok for every later call; scratch for that
+ * many tokens is allocated here, once: about 108 KB a token for the routed
+ * experts and, from 36 tokens on, 6.6 MB and 15.7 KB a token (of at most
+ * 16,384) for the shared expert. */
 NMOE_HIP_API int nmoe_hip_create(int device, int max_tokens, nmoe_hip_ctx **out);
 NMOE_HIP_API void nmoe_hip_destroy(nmoe_hip_ctx *ctx);
 NMOE_HIP_API const char *nmoe_hip_last_error(const nmoe_hip_ctx *ctx);

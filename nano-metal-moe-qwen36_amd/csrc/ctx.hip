@@ -55,11 +55,12 @@ extern "C" int nmoe_hip_create(int device, int max_tokens, nmoe_hip_ctx **out) {
     size_t bytes_act = mt * NMOE_MAX_K * NMOE_INTER * sizeof(float);
     size_t bytes_logits = mt * NMOE_EXPERTS * sizeof(float);
     size_t bytes_idx = mt * NMOE_MAX_K * sizeof(uint32_t);
+    extern size_t nmoe_shared_scratch_bytes(int);
     if (hipMalloc((void **)&ctx->act, bytes_act) != hipSuccess ||
         hipMalloc((void **)&ctx->logits, bytes_logits) != hipSuccess ||
         hipMalloc((void **)&ctx->idx, bytes_idx) != hipSuccess ||
         hipMalloc((void **)&ctx->w, bytes_idx) != hipSuccess ||
-        hipMalloc((void **)&ctx->s_act, mt * NMOE_INTER * sizeof(float)) != hipSuccess ||
+        hipMalloc((void **)&ctx->s_act, nmoe_shared_scratch_bytes(max_tokens)) != hipSuccess ||
         hipMalloc((void **)&ctx->sync, NMOE_SYNC_WORDS * sizeof(uint32_t)) != hipSuccess ||
         hipMemset(ctx->sync, 0, NMOE_SYNC_WORDS * sizeof(uint32_t)) != hipSuccess ||
         hipDeviceSynchronize() != hipSuccess) {

@@ -1876,11 +1876,8 @@ int nmoe_pack_stripe(nmoe_hip_ctx *ctx, int layer) {
 
 /* ------------------------------------------------------------ host */
 
-extern "C" size_t nmoe_shared_mm_bytes(int max_tokens);
-
 extern "C" int nmoe_grouped_init(nmoe_hip_ctx *ctx) {
     const size_t mt = (size_t)ctx->max_tokens, rows = mt * NMOE_MAX_K, places = (size_t)nmoe_work_places((int)rows);
-    const size_t y_bytes = rows * NMOE_HIDDEN * sizeof(float), mm_bytes = nmoe_shared_mm_bytes(ctx->max_tokens);
     ctx->grouped_min_tokens = 8;
     if (hipMalloc((void **)&ctx->g_counts, NMOE_DISPATCH_MAX * NMOE_EXPERTS * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_perm, rows * sizeof(uint32_t)) != hipSuccess ||
@@ -1892,11 +1889,10 @@ extern "C" int nmoe_grouped_init(nmoe_hip_ctx *ctx) {
         hipMalloc((void **)&ctx->g_ahi, rows * NMOE_INTER * sizeof(uint16_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_alo, rows * NMOE_INTER * sizeof(uint16_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_as, rows * (NMOE_INTER / NMOE_GROUP) * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&ctx->g_y, y_bytes + mm_bytes) != hipSuccess ||
+        hipMalloc((void **)&ctx->g_y, rows * NMOE_HIDDEN * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_done, places * sizeof(uint32_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_tags, rows * sizeof(uint64_t)) != hipSuccess)
         return NMOE_HIP_ENOMEM;
-    ctx->s_mm = mm_bytes != 0 ? (uint8_t *)ctx->g_y + y_bytes : NULL; /* (y_bytes is a multiple of 64 KB) */
     ctx->grouped_one_launch = ctx->xcd_placed;
     ctx->skew_tiles = -1;
     /* the dispatch's words start in range (epoch 0, which no launch takes):

@@ -135,8 +135,8 @@ struct nmoe_hip_ctx {
     uint16_t *g_ahi, *g_alo; /* [T*8][512] act (bf16 hi / lo), by permuted row */
     float *g_as;            /* [T*8][8] group sums of act */
     float *g_y;             /* [T*8][2048] per-entry expert outputs */
-    float *s_act;           /* [T][512] shared-expert activations (few tokens) */
-    void *s_mm;             /* the shared expert's matrix-core scratch, after g_y (NULL for contexts of few tokens) */
+    float *s_act;           /* the shared expert's scratch: activations of few tokens, then the matrix-core
+                               launches' (nmoe_shared_scratch_bytes) */
     /* the MoE blocks of the model weights loaded by nmoe_hip_load_model_weights */
     nmoe_hip_moe_block blocks[NMOE_HIP_MAX_LAYERS];
     unsigned char block_set[NMOE_HIP_MAX_LAYERS];

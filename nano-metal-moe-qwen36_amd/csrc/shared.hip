@@ -130,7 +130,7 @@ typedef __attribute__((ext_vector_type(4))) float nmoe_sh_f32x4;
 #define NMOE_SH_GU_G (NMOE_HIDDEN / NMOE_GROUP)
 #define NMOE_SH_DN_G (NMOE_INTER / NMOE_GROUP)
 
-/* The launches' scratch (device): nmoe_shared_init. */
+/* The launches' scratch (device): nmoe_sh_layout. */
 struct nmoe_sh_ws {
     uint4 *wgu;     /* [64 row blocks: gate 0..31, up 32..63][64][64] */
     uint4 *wdn;     /* [128][16][64] */
@@ -170,15 +170,16 @@ __device__ __forceinline__ void nmoe_sh_split3(float v, uint32_t p[3]) {
 /* Blocks 0 .. NMOE_SH_WB - 1: the codes, one wavefront a (row block, 8
  * slices); the next NMOE_SH_SB: scales and biases, 8 a thread; then four
  * blocks for each 16 tokens: planes and group sums, a wavefront 4 slices;
- * then one wavefront a token: the score row. */
+ * then one wavefront a token: the score row.  b0: the first of them this
+ * launch runs (the weights' are done once for all chunks of a call). */
 #define NMOE_SH_WU ((1024 / 16) * (NMOE_SH_GU_SL / 8) + (NMOE_HIDDEN / 16) * (NMOE_SH_DN_SL / 8))
 #define NMOE_SH_WB (NMOE_SH_WU / 4)
 #define NMOE_SH_SB ((1024 * NMOE_SH_GU_G + 2 * NMOE_HIDDEN * NMOE_SH_DN_G) / 8 / 256)
 template <typename XT>
 __global__ void __launch_bounds__(256) nmoe_shared_prep_kernel(nmoe_hip_shared_expert se, nmoe_sh_ws ws, const XT *x,
-                                                               int ntok, int ntb, float *graw) {
+                                                               int ntok, int ntb, int b0, float *graw) {
     constexpr int PL = sizeof(XT) == 2 ? 1 : 3;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, b = blockIdx.x;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, b = blockIdx.x + b0;
     if (b < NMOE_SH_WB) {
         constexpr int GUU = (1024 / 16) * (NMOE_SH_GU_SL / 8);
         const int u = 4 * b + wave;
@@ -497,6 +498,12 @@ __global__ void __launch_bounds__(256, 2) nmoe_shared_mm_kernel(nmoe_sh_ws ws, i
  * 22 at 37. */
 #define NMOE_SHARED_MM_MIN 36
 
+/* Tokens the three launches take at a time, which bounds their scratch (15,680
+ * bytes a token and 6.6 MB of the weights' copies) at 264 MB.  Chunks of 4,096
+ * would take 71 MB, but a call of 4,097 to 16,384 bf16 tokens 4 to 9 % longer
+ * (8,192: 172 and 179 us; fp32 x 229 and 238, 16,384: 528 and 477). */
+#define NMOE_SHARED_CHUNK 16384
+
 /* Scratch of the matrix-core launches, every part a multiple of 1 KB. */
 static size_t nmoe_sh_layout(size_t max_tokens, uint8_t *base, nmoe_sh_ws *ws) {
     const size_t tb = (max_tokens + 15) / 16;
@@ -517,11 +524,14 @@ static size_t nmoe_sh_layout(size_t max_tokens, uint8_t *base, nmoe_sh_ws *ws) {
     return at;
 }
 
-/* Bytes of that scratch; the grouped path's allocation holds it at its end
- * (one allocation more would lengthen the context's creation). */
-extern "C" size_t nmoe_shared_mm_bytes(int max_tokens) {
+/* The shared expert's scratch: the per-token kernels' activations, then, in
+ * contexts of enough tokens, the matrix-core launches'. */
+#define NMOE_SH_ACT_BYTES ((size_t)(NMOE_SHARED_MM_MIN - 1) * NMOE_INTER * sizeof(float))
+static_assert(NMOE_SH_ACT_BYTES % 1024 == 0, "the parts after it stay aligned");
+extern "C" size_t nmoe_shared_scratch_bytes(int max_tokens) {
     nmoe_sh_ws ws;
-    return max_tokens < NMOE_SHARED_MM_MIN ? 0 : nmoe_sh_layout((size_t)max_tokens, NULL, &ws);
+    if (max_tokens < NMOE_SHARED_MM_MIN) return (size_t)max_tokens * NMOE_INTER * sizeof(float);
+    return NMOE_SH_ACT_BYTES + nmoe_sh_layout((size_t)min(max_tokens, NMOE_SHARED_CHUNK), NULL, &ws);
 }
 
 template <int PL, int MB, bool GU>
@@ -544,26 +554,30 @@ static void nmoe_shared_mm_pair(const nmoe_sh_ws &ws, bool bf, int ntok, int ntb
 static void nmoe_shared_mm(nmoe_hip_ctx *ctx, const nmoe_hip_shared_expert *se, const void *x, int x_dtype, int ntok,
                            float *shared_out, float *graw, hipStream_t s) {
     nmoe_sh_ws ws;
-    (void)nmoe_sh_layout((size_t)ctx->max_tokens, (uint8_t *)ctx->s_mm, &ws);
-    const int ntb = (ntok + 15) / 16;
-    const dim3 gp(NMOE_SH_WB + NMOE_SH_SB + 4 * ntb + (ntok + 3) / 4);
+    (void)nmoe_sh_layout((size_t)min(ctx->max_tokens, NMOE_SHARED_CHUNK), (uint8_t *)ctx->s_act + NMOE_SH_ACT_BYTES, &ws);
     const bool bf = x_dtype == NMOE_HIP_BF16;
-    if (bf)
-        hipLaunchKernelGGL(nmoe_shared_prep_kernel<uint16_t>, gp, dim3(256), 0, s, *se, ws, (const uint16_t *)x, ntok,
-                           ntb, graw);
-    else
-        hipLaunchKernelGGL(nmoe_shared_prep_kernel<float>, gp, dim3(256), 0, s, *se, ws, (const float *)x, ntok, ntb,
-                           graw);
-    /* the smallest token tile whose gate/up grid (16 blocks a tile) is one
-     * round of the 256 CUs, then the largest: 16 against 32 and 64 tokens a
-     * tile (fp32 x, us) 26 / 30 / 35 at 251 tokens, 35 / 32 / 35 at 512, 55 /
-     * 44 / 41 at 1,000, 186 / 136 / 121 at 4,096 */
-    if (ntb <= 16)
-        nmoe_shared_mm_pair<1>(ws, bf, ntok, ntb, shared_out, s);
-    else if (ntb <= 32)
-        nmoe_shared_mm_pair<2>(ws, bf, ntok, ntb, shared_out, s);
-    else
-        nmoe_shared_mm_pair<4>(ws, bf, ntok, ntb, shared_out, s);
+    for (int t0 = 0; t0 < ntok; t0 += NMOE_SHARED_CHUNK) {
+        const int n = min(ntok - t0, NMOE_SHARED_CHUNK), ntb = (n + 15) / 16;
+        const int b0 = t0 == 0 ? 0 : NMOE_SH_WB + NMOE_SH_SB;
+        const dim3 gp(NMOE_SH_WB + NMOE_SH_SB - b0 + 4 * ntb + (n + 3) / 4);
+        float *so = shared_out + (size_t)t0 * NMOE_HIDDEN;
+        if (bf)
+            hipLaunchKernelGGL(nmoe_shared_prep_kernel<uint16_t>, gp, dim3(256), 0, s, *se, ws,
+                               (const uint16_t *)x + (size_t)t0 * NMOE_HIDDEN, n, ntb, b0, graw + t0);
+        else
+            hipLaunchKernelGGL(nmoe_shared_prep_kernel<float>, gp, dim3(256), 0, s, *se, ws,
+                               (const float *)x + (size_t)t0 * NMOE_HIDDEN, n, ntb, b0, graw + t0);
+        /* the smallest token tile whose gate/up grid (16 blocks a tile) is one
+         * round of the 256 CUs, then the largest: 16 against 32 and 64 tokens a
+         * tile (fp32 x, us) 26 / 30 / 35 at 251 tokens, 35 / 32 / 35 at 512, 55
+         * / 44 / 41 at 1,000, 186 / 136 / 121 at 4,096 */
+        if (ntb <= 16)
+            nmoe_shared_mm_pair<1>(ws, bf, n, ntb, so, s);
+        else if (ntb <= 32)
+            nmoe_shared_mm_pair<2>(ws, bf, n, ntb, so, s);
+        else
+            nmoe_shared_mm_pair<4>(ws, bf, n, ntb, so, s);
+    }
 }
 
 int nmoe_check_x(nmoe_hip_ctx *ctx, const void *x, int x_dtype, int ntok);

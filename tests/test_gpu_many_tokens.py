@@ -1,6 +1,8 @@
 """GPU: the many-token forms of the shared expert and the routers and the
 grouped experts' work list, through the C ABI, at the sizes where a tile, a
 grid, a piece or a dispatch rule ends."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -109,6 +111,57 @@ def test_shared_expert_place_in_the_call(ctx, nh, xdt, ntok):
     for so, gr in got[1:]:
         np.testing.assert_array_equal(so, got[0][0])
         np.testing.assert_array_equal(gr, got[0][1])
+
+
+@pytest.mark.parametrize("xdt,ntok", [("f32", 16389), ("bf16", 16428)])
+def test_shared_expert_chunks(nh, xdt, ntok):
+    """A call of more tokens than the matrix-core launches take at a time: the
+    tokens around the seam, and the last ones, bit for bit those of a short
+    call's matrix form; the score of the first tokens bit for bit the
+    per-token kernels'; nothing written past the last token."""
+    rng = np.random.default_rng(ntok)
+    with nh.Context(0, max_tokens=ntok) as c:
+        t = [q4_tensor(rng, r, k, s, 1) for r, k, s in
+             ((512, 2048, 0.004), (512, 2048, 0.004), (2048, 512, 0.008), (1, 2048, 0.004))]
+        desc = nh.Context.shared_expert_desc(*(device_copy(c, q, 1) for q in t))
+        _, dx, dt = tokens(rng, c, nh, xdt, ntok)
+        row = 8192 if dt == nh.F32 else 4096
+
+        def run(first, n):
+            so, gr = c.to_device(np.full((n + 1, 2048), 7.5, np.float32)), c.to_device(np.full(n + 1, 7.5, np.float32))
+            c._check(c.shared_expert(desc, dx.ptr + first * row, dt, n, so, gr))
+            so, gr = so.download(np.uint32, (n + 1, 2048)), gr.download(np.uint32, n + 1)
+            assert (so[n].view(np.float32) == 7.5).all() and gr[n:].view(np.float32)[0] == 7.5
+            return so[:n], gr[:n]
+
+        so, gr = run(0, ntok)
+        for first, n in ((0, 36), (ntok - 97, 97), (ntok - 44, 44)):
+            part, pg = run(first, n)
+            np.testing.assert_array_equal(so[first:first + n], part)
+            np.testing.assert_array_equal(gr[first:first + n], pg)
+        np.testing.assert_array_equal(gr[:35], run(0, 35)[1])
+
+
+def test_context_scratch_of_many_tokens(nh):
+    """What a context takes a token beyond 16,384: the routed experts' scratch
+    (108,132 bytes), none for the shared expert, whose own is bounded."""
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l) if nh.lib() else None
+    hip = ctypes.CDLL(path)
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    used = []
+    for n in (16384, 65536):
+        c = nh.Context(0, max_tokens=n)
+        after = free()
+        c.close()
+        used.append(free() - after)
+    per = (used[1] - used[0]) / (65536 - 16384)
+    print(f"[scratch] {used} bytes, {per:.0f} a token")
+    assert per < 108132 + 1000  # the allocations' granules
 
 
 # one row a wavefront for few terms, then tiles of 16 x 16, 32 x 32 (from 513
