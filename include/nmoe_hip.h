@@ -135,16 +135,19 @@ NMOE_HIP_API int nmoe_hip_check_device_status(nmoe_hip_ctx *ctx);
 /* NMOE_HIP_OPT_GROUPED_ONE_LAUNCH (default 1 where the device deals the
  * blocks of a launch round-robin over its 8 dies, checked at create): the
  * grouped path runs gate/up and down in one launch, each down tile starting
- * once its expert's gate/up tiles are done (a bounded wait); 0 runs them as
+ * once its piece's gate/up tiles are done (a bounded wait); 0 runs them as
  * two launches.  The results are the same to the grouped path's
  * tolerance. */
 #define NMOE_HIP_OPT_GROUPED_ONE_LAUNCH 8
-/* NMOE_HIP_OPT_SKEW_TILES (value = expert rank 0..255, by entries, most
- * first; for tests of the failure path): the next one-launch grouped call
- * starts that rank's count of finished gate/up tiles at an impossible
- * value, so its down tiles find the count wrong, as they would had the
- * tiles run on another die: the call's outputs are NaN and
- * nmoe_hip_check_device_status returns NMOE_HIP_ETIMEDOUT.  Once. */
+/* NMOE_HIP_OPT_SKEW_TILES (value = work place 0..255; for tests of the
+ * failure path): the grouped path's work list holds every expert's entries
+ * in pieces of up to 64, whole ones first, then by entries; a call has 256
+ * places and one for every 64 entries, some without a piece.  The next
+ * one-launch grouped call starts that place's count of finished gate/up
+ * tiles at an impossible value, so its down tiles find the count wrong, as
+ * they would had the tiles run on another die: the call's outputs are NaN
+ * and nmoe_hip_check_device_status returns NMOE_HIP_ETIMEDOUT.  Once; a
+ * place without a piece has no tiles, and nothing fails. */
 #define NMOE_HIP_OPT_SKEW_TILES 9
 NMOE_HIP_API int nmoe_hip_set_option(nmoe_hip_ctx *ctx, int option, int value);
 

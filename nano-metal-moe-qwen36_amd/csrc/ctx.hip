@@ -138,7 +138,7 @@ extern "C" int nmoe_hip_set_option(nmoe_hip_ctx *ctx, int option, int value) {
     }
     if (option == NMOE_HIP_OPT_SKEW_TILES) {
         if (value < 0 || value >= NMOE_EXPERTS)
-            return nmoe_fail(ctx, NMOE_HIP_EINVAL, "expert rank %d outside 0..%d", value, NMOE_EXPERTS - 1);
+            return nmoe_fail(ctx, NMOE_HIP_EINVAL, "work place %d outside 0..%d", value, NMOE_EXPERTS - 1);
         ctx->skew_tiles = value;
         return NMOE_HIP_OK;
     }

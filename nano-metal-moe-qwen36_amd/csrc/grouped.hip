@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(256) nmoe_grouped_prep_kernel(const uint32_t *
      * at once by every block) */
     const uint32_t epoch = ROUTED || MULTI ? nmoe_ld_u32_dev(sync + NMOE_SYNC_PREP_EPOCH) + 1u : 0u;
     /* the one-launch GEMM's tile counts start from 0 (plain stores: the next
-     * launch on the stream sees them); rank `skew` (a test of the failure
+     * launch on the stream sees them); place `skew` (a test of the failure
      * path) from a count no tiles can reach */
     if (done != NULL && b == 0)
         for (int i = threadIdx.x; i < ne; i += 256) done[i] = i == skew ? 0x8000u : 0u;

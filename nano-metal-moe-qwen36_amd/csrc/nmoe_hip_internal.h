@@ -122,7 +122,7 @@ struct nmoe_hip_ctx {
     /* grouped (matrix-core) path for many tokens, sized for max_tokens */
     int grouped_min_tokens; /* NMOE_HIP_OPT_GROUPED_MIN_TOKENS */
     int grouped_one_launch; /* NMOE_HIP_OPT_GROUPED_ONE_LAUNCH */
-    int skew_tiles;         /* NMOE_HIP_OPT_SKEW_TILES: rank, or -1 */
+    int skew_tiles;         /* NMOE_HIP_OPT_SKEW_TILES: work place, or -1 */
     uint32_t *g_done;       /* [places] the one-launch form's gate/up tiles done per work place */
     uint64_t *g_tags;       /* [T*8] routed entries of the preparation launch: epoch << 32 | expert */
     uint64_t *g_counts;     /* [64][256] per-slice expert histograms, each word epoch << 32 | count */

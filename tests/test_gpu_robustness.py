@@ -155,9 +155,9 @@ def test_sync_check_returns_etimedout(nh):
 
 
 def test_grouped_one_launch_wrong_tile_count_poisons_and_recovers(nh):
-    """The one-launch grouped form: a down tile checks that its expert's
+    """The one-launch grouped form: a down tile checks that its piece's
     gate/up tiles are all counted, each from this block's die.  With the
-    count of expert rank 0 started at an impossible value
+    count of work place 0 started at an impossible value
     (NMOE_HIP_OPT_SKEW_TILES), its down tiles find it wrong: the call's
     outputs are NaN and the status reports ETIMEDOUT; the next call is the
     same bits as the two-launch form's."""
@@ -170,7 +170,7 @@ def test_grouped_one_launch_wrong_tile_count_poisons_and_recovers(nh):
         idx = np.zeros((ntok, 8), np.uint32)
         for t in range(ntok):
             idx[t, :k] = rng.choice(256, k, replace=False)
-        idx[:40, 0] = 7  # rank 0: expert 7 with 40 entries
+        idx[:40, 0] = 7  # place 0: expert 7 with 40 entries
         w = rng.dirichlet(np.ones(k), size=ntok).astype(np.float32)
         x = rng.standard_normal((ntok, 2048)).astype(np.float32)
         h = rng.standard_normal((ntok, 2048)).astype(np.float32)
@@ -194,6 +194,45 @@ def test_grouped_one_launch_wrong_tile_count_poisons_and_recovers(nh):
         np.testing.assert_array_equal(run().view(np.uint32), want.view(np.uint32))
         assert ctx.device_status() == nh.OK
         assert ctx.set_option(nh.OPT_SKEW_TILES, 256) == nh.EINVAL
+
+
+def test_grouped_wrong_tile_count_of_one_piece(nh):
+    """An expert of more than 64 entries has a work place for each piece: the
+    count of any one of them started wrong, or of a short piece, fails the
+    call, and the call after it is right again; a place without a piece has no
+    tiles, and nothing fails."""
+    rng = np.random.default_rng(79)
+    ntok, k, layer, bits = 130, 3, 4, 4
+    with nh.Context(0, max_tokens=ntok) as ctx:
+        if not ctx.set_grouped_one_launch(True):
+            pytest.skip("the one-launch form needs the round-robin die placement")
+        ctx.synth_layer(layer, bits, 11, 0.02)
+        idx = np.zeros((ntok, 8), np.uint32)
+        # pieces of 64, 64 and 2 (experts 7 and 40) and of 43 or 44 (9 .. 11)
+        idx[:, 0], idx[:, 1], idx[:, 2] = 7, 9 + np.arange(ntok) % 3, 40
+        w = rng.dirichlet(np.ones(8), size=ntok).astype(np.float32)
+        d = [ctx.to_device(a) for a in (rng.standard_normal((ntok, 2048)).astype(np.float32), idx, w,
+                                        rng.standard_normal((ntok, 2048)).astype(np.float32))]
+        out = ctx.alloc(ntok * 8192)
+
+        def run():
+            ctx._check(ctx.experts(bits, layer, d[0], nh.F32, ntok, k, d[1], d[2], d[3], out))
+            return out.download(np.float32, (ntok, 2048)), ctx.device_status()
+
+        want, status = run()
+        assert status == nh.OK and np.isfinite(want).all()
+        # the second pieces of 7 and 40, one of 9 .. 11, and (rounds of eight go 0 .. 7, then 15 .. 8) the last piece
+        for place in (1, 3, 5, 15, 255):
+            ctx._check(ctx.set_option(nh.OPT_SKEW_TILES, place))
+            bad, status = run()
+            if place == 255:
+                assert status == nh.OK
+                np.testing.assert_array_equal(bad.view(np.uint32), want.view(np.uint32))
+            else:
+                assert status == nh.ETIMEDOUT and np.isnan(bad).all(), place
+            again, status = run()
+            assert status == nh.OK
+            np.testing.assert_array_equal(again.view(np.uint32), want.view(np.uint32))
 
 
 def test_grouped_routed_after_aborted_launch(nh):
