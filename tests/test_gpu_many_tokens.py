@@ -66,8 +66,8 @@ def tokens(rng, ctx, nh, xdt, ntok):
 def test_shared_expert_many_tokens(ctx, nh, xdt, ntok):
     """shared_out and the score against the products in 64 bits (relative L2
     within 1e-6: fp32 sums of 2,048 and 512 terms, each rounding 2^-24, stay
-    below 5e-7), a few tokens against the oracle, and nothing written past
-    the last token."""
+    below 5e-7), a few tokens against the oracle, every token's score bit for
+    bit the per-token kernels', and nothing written past the last token."""
     rng = np.random.default_rng(1000 + ntok)
     t = {n: q4_tensor(rng, r, c, s, 1) for n, (r, c, s) in
          {"gate": (512, 2048, 0.004), "up": (512, 2048, 0.004), "down": (2048, 512, 0.008),
@@ -91,6 +91,11 @@ def test_shared_expert_many_tokens(ctx, nh, xdt, ntok):
     pick = np.unique([0, ntok // 2, ntok - 1])
     want_so, want_gr = B.shared_expert({n: t[n] for n in t}, x[pick])
     assert rel(got[pick], want_so) < 2e-6 and rel(got_g[pick], want_gr) < 2e-6
+    few = ctx.alloc(ntok * 4)
+    for t0 in range(0, ntok, 32):
+        ctx._check(ctx.shared_expert(desc, dx.ptr + t0 * 2048 * (4 if dt == nh.F32 else 2), dt, min(32, ntok - t0), so,
+                                     few.ptr + 4 * t0))
+    np.testing.assert_array_equal(got_g[:ntok].view(np.uint32), few.download(np.uint32, ntok))
 
 
 @pytest.mark.parametrize("xdt,ntok", [("f32", 67), ("bf16", 300)])
@@ -260,23 +265,26 @@ def test_router_q4_extreme_products(ctx, nh, xdt, ntok):
 
 
 # entries an expert gets: either side of a 16-entry row block and of one, two
-# and three 64-entry pieces; one expert only; few experts of many pieces.  A
-# third of the tokens also have an entry on an expert of few entries; slots
-# left over hold indexes outside the layer
+# and three 64-entry pieces; one expert only; few experts of many pieces, on
+# either side of the most entries one launch takes (8,192); every expert with
+# a piece of 32, the most pieces of more than 16 entries.  A third of the
+# tokens also have an entry on an expert of few entries; slots left over hold
+# indexes outside the layer
 @pytest.mark.parametrize("bits,xdt,counts,ntok", [
     (4, "f32", [63, 64, 65, 127, 128, 129, 16, 17, 1, 2], 129), (2, "bf16", [64, 128, 192, 193, 15, 48, 49], 193),
-    (4, "bf16", [200], 200), (2, "f32", [1025, 1024, 961, 960, 449], 1025)])
+    (4, "bf16", [200], 200), (2, "f32", [1025, 1024, 961, 960, 449], 1025), (4, "bf16", [1024, 1000, 961, 449], 1024),
+    (4, "f32", [32] * 256, 1024), (2, "bf16", [32] * 256, 1024)])
 def test_grouped_pieces(nh, bits, xdt, counts, ntok):
-    """The grouped path (in one launch and in two: the same bits) against the
-    per-token kernels of the same call, relative L2 within 1e-4 as the
-    path's act planes (2^-17 a term) and fp32 sums allow, every token held
-    to 1e-3, and nothing written past the last token."""
+    """The grouped path (in one launch, up to 8,192 entries, and in two: the
+    same bits) against the per-token kernels of the same call, relative L2
+    within 1e-4 as the path's act planes (2^-17 a term) and fp32 sums allow,
+    every token held to 1e-3, and nothing written past the last token."""
     rng = np.random.default_rng(len(counts) + ntok)
     slots = np.full((ntok, 8), 0xFFFFFFFF, np.uint32)
     fill = np.zeros(ntok, int)
-    for e, n in enumerate(counts):  # expert 11 e: n different tokens, the emptiest first
+    for e, n in enumerate(counts):  # expert 11 e mod 256: n different tokens, the emptiest first
         for t in np.argsort(fill + rng.random(ntok) * 0.5)[:n]:
-            slots[t, fill[t]] = 11 * e
+            slots[t, fill[t]] = 11 * e % 256
             fill[t] += 1
     if len(counts) > 1:
         for t in range(0, ntok, 3):
@@ -300,6 +308,13 @@ def test_grouped_pieces(nh, bits, xdt, counts, ntok):
             assert (o[ntok] == 7.5).all()
             got.append(o[:ntok].astype(np.float64) - h)
         assert c.device_status() == nh.OK
+        # a wrong tile count fails a call in one launch alone: which of the forms ran above
+        c.set_grouped_min_tokens(8)
+        if c.set_grouped_one_launch(True):
+            assert len(got) == 3
+            c._check(c.set_option(nh.OPT_SKEW_TILES, 0))
+            c._check(c.experts(bits, 1, dx, dt, ntok, 8, di, dw, dh, out))
+            assert c.device_status() == (nh.ETIMEDOUT if ntok * 8 <= 8192 else nh.OK)
     finally:
         c.close()
     want = got.pop()
