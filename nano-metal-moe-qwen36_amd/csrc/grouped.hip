@@ -160,12 +160,6 @@ __device__ __forceinline__ uint32_t nmoe_bf16_rne(float f) {
  * even), one instruction. */
 __device__ __forceinline__ uint32_t nmoe_bf16_cvt(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
-/* A raw buffer resource over p: base in scalar registers, range 2 GB (the
- * offsets used stay far inside the allocation), untyped access. */
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t nmoe_buffer(void *p) {
-    return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, 0x7fffffff, 0x00020000);
-}
-
 /* An LDS address as the direct global->LDS loads take it. */
 typedef __attribute__((address_space(3))) void nmoe_lds_void;
 
@@ -1114,7 +1108,7 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
      * matrix cmat (gate for the first half of the wavefronts, up for the
      * second) */
     const int cmat = wave / (NW / 2);
-    const __amdgpu_buffer_rsrc_t crs = nmoe_buffer((void *)(ex + (cmat == 0 ? L::gate_w : L::up_w))); /* stripe-major */
+    const __amdgpu_buffer_rsrc_t crs = nmoe_buffer(ex + (cmat == 0 ? L::gate_w : L::up_w)); /* stripe-major */
     const uint16_t *bias[2] = {(const uint16_t *)(ex + L::gate_b) + (size_t)nt * NT * G,
                                (const uint16_t *)(ex + L::up_b) + (size_t)nt * NT * G};
 
@@ -1151,7 +1145,7 @@ __device__ __forceinline__ void nmoe_gu_tile(const uint8_t *pack, const uint16_t
 #pragma unroll
     for (int i = 0; i < AI; i++)
         row_off[i] = s_tok[8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3)] * (uint32_t)(NMOE_HIDDEN * 2);
-    const __amdgpu_buffer_rsrc_t xpl[2] = {nmoe_buffer((void *)xhi), nmoe_buffer((void *)xlo)};
+    const __amdgpu_buffer_rsrc_t xpl[2] = {nmoe_buffer(xhi), nmoe_buffer(xlo)};
     auto issue = [&](int gs, int st) {
 #pragma unroll
         for (int pl = 0; pl < XPL; pl++)
@@ -1466,7 +1460,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint8_t *ex = pack + (size_t)e * L::expert_size;
     const int rt0 = (NT / NW) * wave + col; /* tile row of column block nb: rt0 + 16 nb */
-    const __amdgpu_buffer_rsrc_t crs = nmoe_buffer((void *)(ex + L::down_w)); /* stripe-major */
+    const __amdgpu_buffer_rsrc_t crs = nmoe_buffer(ex + L::down_w); /* stripe-major */
     const uint16_t *bias = (const uint16_t *)(ex + L::down_b) + (size_t)nt * NT * G;
 
     /* the tile in one form: n <= MCH entries, GPS groups a ring step */
@@ -1501,7 +1495,7 @@ __device__ __forceinline__ void nmoe_dn_tile(const uint8_t *pack, const uint16_t
     for (int i = 0; i < AI; i++)
         row_off[i] = (p0 + min((uint32_t)(8 * ((wave + NW * i) % (MCH / 8)) + (lane >> 3)), n - 1)) *
                      (uint32_t)(NMOE_INTER * 2);
-    const __amdgpu_buffer_rsrc_t apl[2] = {nmoe_buffer((void *)ahi), nmoe_buffer((void *)alo)};
+    const __amdgpu_buffer_rsrc_t apl[2] = {nmoe_buffer(ahi), nmoe_buffer(alo)};
     /* a stage's act rows (2 AI loads) and its codes (CP::PER_WAVE loads) */
     auto issue_a = [&](int gs, int st) {
 #pragma unroll

@@ -126,10 +126,6 @@ typedef __attribute__((ext_vector_type(4))) float nmoe_rt_f32x4;
 typedef __attribute__((ext_vector_type(16))) float nmoe_rt_f32x16;
 typedef __attribute__((ext_vector_type(2))) uint16_t nmoe_rt_u16x2;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t nmoe_rt_buffer(const void *p) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, 0x7fffffff, 0x00020000);
-}
-
 /* Registers v[0..3] (elements) over the lane rows 0..3 (segments) become
  * registers (segments) over lane rows (elements). */
 __device__ __forceinline__ void nmoe_rt_transpose4(float v[4]) {
@@ -191,7 +187,7 @@ __global__ void __launch_bounds__(512) nmoe_router_mm_kernel(const void *__restr
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, kb = lane >> 4;
     const int t0 = 16 * MT * (int)blockIdx.y, e0 = 16 * NT * (int)blockIdx.x;
-    const __amdgpu_buffer_rsrc_t xr = nmoe_rt_buffer(x), wr = nmoe_rt_buffer(w);
+    const __amdgpu_buffer_rsrc_t xr = nmoe_buffer(x), wr = nmoe_buffer(w);
     uint32_t xoff[MT], woff[NT]; /* bytes; rows past the end read the last one and are not stored */
 #pragma unroll
     for (int m = 0; m < MT; m++) xoff[m] = (uint32_t)(min(t0 + 16 * m + r, ntok - 1) * NMOE_HIDDEN + 512 * kb) * (uint32_t)sizeof(XT);

@@ -147,11 +147,7 @@ __device__ __forceinline__ nmoe_sh_f32x4 nmoe_sh_mfma(uint4 a, uint4 b, nmoe_sh_
                                                    __builtin_bit_cast(nmoe_sh_bf16x8, b), c, 0, 0, 0);
 }
 
-/* A raw buffer resource over p (base in scalar registers, range 2 GB; every
- * offset used stays inside the allocation) and a 16-byte load from it. */
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t nmoe_sh_buffer(void *p) {
-    return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, 0x7fffffff, 0x00020000);
-}
+/* A 16-byte load from a buffer resource. */
 __device__ __forceinline__ uint4 nmoe_sh_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
     return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
 }
@@ -324,8 +320,8 @@ __global__ void __launch_bounds__(256, 2) nmoe_shared_mm_kernel(nmoe_sh_ws ws, i
     /* Loads through raw buffer resources: one scalar offset a tile and slice
      * on top of the lane's 16 bytes, and (as these are intrinsics) they stay
      * where the ring issues them. */
-    const __amdgpu_buffer_rsrc_t ar = nmoe_sh_buffer(GU ? (void *)ws.xp : (void *)ws.ap),
-                                 br = nmoe_sh_buffer(GU ? (void *)ws.wgu : (void *)ws.wdn);
+    const __amdgpu_buffer_rsrc_t ar = nmoe_buffer(GU ? ws.xp : ws.ap),
+                                 br = nmoe_buffer(GU ? ws.wgu : ws.wdn);
     const uint16_t *sc = GU ? ws.sgu : ws.sdn, *bs = sc + (GU ? 1024 : NMOE_HIDDEN) * G;
     uint32_t aoff[MB][PL], boff[4]; /* bytes */
 #pragma unroll
@@ -353,7 +349,7 @@ __global__ void __launch_bounds__(256, 2) nmoe_shared_mm_kernel(nmoe_sh_ws ws, i
 #pragma unroll
         for (int j = 0; j < 4; j++) b[buf][j] = nmoe_sh_load(br, 16u * lane, boff[j] + 1024u * (uint32_t)s);
     };
-    const __amdgpu_buffer_rsrc_t sr = nmoe_sh_buffer((void *)sc);
+    const __amdgpu_buffer_rsrc_t sr = nmoe_buffer(sc);
     auto load_s = [&](int j, int g) { /* the scales of groups g and g + 1 (from the wavefront's first) */
         return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(sr, 2 * G * col, 32 * G * rb[j] + s0 + 2 * g, 0);
     };
