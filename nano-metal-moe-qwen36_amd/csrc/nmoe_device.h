@@ -237,12 +237,6 @@ __device__ __forceinline__ void nmoe_unpack_bf16x8(uint4 v, float out[8]) {
     }
 }
 
-/* A raw buffer resource over p: base in scalar registers, range 2 GB (every
- * offset used stays inside the allocation), untyped access. */
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t nmoe_buffer(const void *p) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, 0x7fffffff, 0x00020000);
-}
-
 /* n consecutive activations starting at column c0, as fp32. */
 template <typename XT>
 __device__ __forceinline__ void nmoe_load_cols(const XT *x, int c0, int n, float *out);

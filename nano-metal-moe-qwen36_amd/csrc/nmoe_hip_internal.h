@@ -177,4 +177,10 @@ __device__ __forceinline__ uint32_t nmoe_f32_to_bf16_bits(float f) {
     return (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
 }
 
+/* A raw buffer resource over p: base in scalar registers, range 2 GB (every
+ * offset used stays inside the allocation), untyped access. */
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t nmoe_buffer(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, 0x7fffffff, 0x00020000);
+}
+
 #endif
