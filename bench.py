@@ -518,8 +518,8 @@ def run_grouped(pool, args, workload: str, NLg: int = 8) -> dict:
         touched.append(len(np.unique(top)))
     IDX, WT, OUT = ctx.alloc(ntok * 32), ctx.alloc(ntok * 32), ctx.alloc(ntok * 2048 * 4)
     # the library runs gate/up and down in one launch where the device allows
-    # it and the experts average at most half a 64-entry pass (one pass lane:
-    # ntok * k <= 8192), else in two
+    # it and the experts average at most half a 64-entry piece (ntok * k <=
+    # 8192), else in two
     one = args.grouped_launches == 1 and ctx.set_grouped_one_launch(True) and ntok * k <= 8192
     if args.grouped_launches == 2:
         ctx.set_grouped_one_launch(False)

@@ -73,9 +73,10 @@ __host__ __device__ constexpr int nmoe_dispatch_blocks(int n) {
  * This many places (a multiple of 8; those without a piece hold no entries)
  * cover any routing of n entries, and the GEMM grids are sized for them.  A
  * block runs one piece: an expert of many entries does not run its pieces one
- * after the other in the blocks of its tiles (4,096 tokens, fp32 x, q4, the
- * GEMMs: 1.27 ms with two sets of blocks a tile, 0.97 so; 1,000 tokens, q2,
- * 245 and 212 us).  Below 256 entries fewer places would do, but the down
+ * after the other in the blocks of its tiles (a whole layer's calls, shared
+ * expert, router and combine among them, 4,096 tokens, fp32 x, q4: 1.27 ms
+ * with two sets of blocks a tile, 0.97 so; 1,000 tokens, q2, 245 and 212 us).
+ * Below 256 entries fewer places would do, but the down
  * tiles of the one-launch form then start too early (13 tokens 3 % slower). */
 __host__ __device__ constexpr int nmoe_work_places(int n) {
     return (NMOE_EXPERTS + n / NMOE_MCHUNK + 7) / 8 * 8;
@@ -1872,6 +1873,12 @@ int nmoe_pack_stripe(nmoe_hip_ctx *ctx, int layer) {
 
 extern "C" int nmoe_grouped_init(nmoe_hip_ctx *ctx) {
     const size_t mt = (size_t)ctx->max_tokens, rows = mt * NMOE_MAX_K, places = (size_t)nmoe_work_places((int)rows);
+    /* 8 tokens: drawn when the per-token kernels took longer.  Now they are
+     * ahead of the grouped path to about 16 tokens of 8 experts and further
+     * with fewer (us a call, per-token and grouped, bf16 x: q4, k = 8, 33.9
+     * and 42.0 at 8 tokens, 54.5 and 56.0 at 16, 64.7 and 58.9 at 20; q2 28.9
+     * and 38.6, 44.8 and 49.6, 53.3 and 49.6; k = 6, q4, 60.8 and 58.5 at 24;
+     * k = 1 18.9 and 30.8 there) */
     ctx->grouped_min_tokens = 8;
     if (hipMalloc((void **)&ctx->g_counts, NMOE_DISPATCH_MAX * NMOE_EXPERTS * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc((void **)&ctx->g_perm, rows * sizeof(uint32_t)) != hipSuccess ||
@@ -1944,7 +1951,14 @@ static int nmoe_grouped_run(nmoe_hip_ctx *ctx, const uint8_t *pack, const void *
     const int ne = nmoe_work_places(ntok * k);
     /* gate/up and down in one launch where the blocks' dies are known, up to
      * 32 entries an expert on average; beyond, the one-launch form's smaller
-     * down tiles cost more than the overlap gains */
+     * down tiles cost more than the overlap gains (one and two launches, us a
+     * call, q4, bf16 x: 178.5 and 170.8 at 9,600 entries, 274 and 263 at
+     * 16,384).  The line was drawn when an expert's pieces ran one after the
+     * other; on the work list the two forms are level at 2,048 entries (113.4
+     * and 113.1; fp32 x 125.4 and 123.2) and two launches ahead from about
+     * 4,096 with even routing (129.6 and 128.0, at 8,192 167.3 and 161.2; q2
+     * 111.6 and 108.5, 153.8 and 147.2), with skewed routing and bf16 x not up
+     * to the line (183.9 and 190.4; q2 159.8 and 160.6) */
     const bool one = ctx->grouped_one_launch && ctx->xcd_placed && (long)ntok * k <= (long)NMOE_EXPERTS * NMOE_MCHUNK / 2;
     uint32_t *done = one ? ctx->g_done : NULL;
     const int skew = one ? ctx->skew_tiles : -1;

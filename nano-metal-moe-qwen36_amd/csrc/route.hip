@@ -172,13 +172,16 @@ struct nmoe_rt_raw {
 
 /* MT x NT tiles of 16 tokens x 16 experts a block of eight wavefronts.
  * Bound: bf16 router, the fp32 MFMA rate (128 fmas a clock a CU: 28 us for
- * 4,096 tokens) and the lines of w and x (a lane reads 32 or 64 bytes of a
- * row at a time; one chain at a time, 16 or 32, took 63 against 51 us); q4
- * router, fp32 MFMAs and vector instructions, which do not overlap on this
- * part (2 MFMAs and 16 fma + 16 add a four-column step with fp32 x: 192
- * clocks of the 220 measured).  4,096 tokens, one-row-a-wavefront kernels
+ * 4,096 tokens, matrix cores busy 41 % of the launch with fp32 x, 46 % with
+ * bf16 x) and the lines of w and x (a lane reads 32 or 64 bytes of a row at a
+ * time; one chain at a time, 16 or 32, took 63 against 51 us; each die reads
+ * all of x, 328 MB of 34 in all with fp32 x); q4 router, fp32 MFMAs and vector
+ * instructions, which do not overlap on this part (the counter of cycles with
+ * both is 0; together they take 96 % of the launch's cycles with fp32 x, 93 %
+ * with bf16 x; 2 MFMAs and 16 fma + 16 add a four-column step with fp32 x:
+ * 192 clocks of the 220 measured).  4,096 tokens, one-row-a-wavefront kernels
  * against this (us): bf16 router 292 -> 61 (fp32 x), 166 -> 51 (bf16 x); q4
- * router 301 -> 201, 227 -> 135. */
+ * router 301 -> 202, 227 -> 145. */
 template <bool Q4, typename XT, int MT, int NT>
 __global__ void __launch_bounds__(512) nmoe_router_mm_kernel(const void *__restrict__ w, const uint16_t *__restrict__ sc,
                                                              const uint16_t *__restrict__ bi, const XT *__restrict__ x,

@@ -294,7 +294,8 @@ __global__ void __launch_bounds__(256) nmoe_shared_prep_kernel(nmoe_hip_shared_e
  * 4 (down) slices long and nothing is shared, or waited for, before the end.
  * Operands go straight from their operand-order copies into registers.
  * Bound: the two operands' way from the L2 (64 x 64 tiles read 16 KB of them
- * for 32 MFMAs), at 2,048 and more tokens; the launches and one chain's
+ * for 32 MFMAs), at 2,048 and more tokens (4,096, fp32 x: gate/up's matrix
+ * cores busy 35 % of the launch, no unit 57 %); the launches and one chain's
  * latency below.  Measured (three launches, us, fp32 x / bf16 x, against the
  * per-token kernels): 64 tokens 22 / 21 from 32 / 31, 251 tokens 26 / 25 from
  * 107 / 96, 1,000 tokens 41 / 35 from 415 / 367, 4,096 tokens 121 / 94 from
@@ -419,7 +420,7 @@ __global__ void __launch_bounds__(256, 2) nmoe_shared_mm_kernel(nmoe_sh_ws ws, i
                 if (GU) {
                     /* sum_g c_g xs_g on the matrix cores, both factors as
                      * three bf16 parts: the products down to 2^-24, smallest
-                     * first (c = 0, the converter's usual b = -8 s, gives 0) */
+                     * first */
                     nmoe_sh_f32x4 cc = zero;
                     uint4 xv[3], cv[3];
 #pragma unroll

@@ -1,7 +1,7 @@
 """The context's entry points captured into HIP graphs and replayed, as a
 serving loop would: nmoe_moe_experts_from_logits (the grouped path, with
-gate/up and down in one launch and in two, and with two pass lanes) and
-nmoe_moe_layer (the fused single-token launch).  Capture is global-mode, so
+gate/up and down in one launch and in two, and with several dispatch slices)
+and nmoe_moe_layer (the fused single-token launch).  Capture is global-mode, so
 any call illegal under capture fails it; every captured node must be a
 kernel (no memset or copy nodes).  Each replay runs on new inputs written
 into the captured buffers, with eager calls of the same entry point in
@@ -64,8 +64,8 @@ def _same(got, want, what):
 
 @pytest.mark.parametrize("bits,ntok,one", [(4, 64, True), (4, 64, False), (2, 64, True), (4, 1200, True)])
 def test_grouped_from_logits_graph_replays(nh, bits, ntok, one):
-    """64 tokens: one pass lane (gate/up and down in one launch, or in two);
-    1200 tokens: two pass lanes and 8 dispatch slices (two launches)."""
+    """64 tokens: gate/up and down in one launch, or in two; 1200 tokens: 9,600
+    entries, 16 dispatch slices, two launches."""
     hp = hip()
     k, layer = 8, 6
     rng = np.random.default_rng(900 + bits + ntok)
